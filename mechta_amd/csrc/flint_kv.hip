@@ -19,6 +19,7 @@
 // flint_attn.wgsl:241-257: the sink joins the maximum and the sum, never the output) and normalizes.
 #include "flint_internal.h"
 #include "mkv_device.h"
+#include "mkv_rows.h"
 
 namespace mkv {
 namespace flint {
@@ -693,7 +694,8 @@ __global__ void __launch_bounds__(64) fl_rope(int heads, const float* __restrict
     out[h0 + i + 64] = x0 * sn + x1 * cs;
 }
 
-// Store layout <-> the reference's rows [row][kvh][128] for rows [r0, r1) of one layer's K or V.
+// Store layout <-> the reference's rows [row][kvh][128] for rows [r0, r1) of one layer's K or V, where the rows are not
+// 16-byte aligned (the others take rows_tile, mkv_rows.h).
 template <typename E, int DIR>  // DIR 0: store -> rows, 1: rows -> store
 __global__ void __launch_bounds__(256) fl_rows(E* __restrict__ plane, size_t plane_elems, E* __restrict__ rowsbuf,
                                                int r0, int r1, int which) {
@@ -1132,6 +1134,10 @@ hipError_t launch_rows(int fmt, void* plane, int rows, int which, int r0, int r1
     const dim3 grid((unsigned)((total + 255) / 256));
     const size_t pe = (size_t)rows * HD;
     const Launch L{st};
+    if ((uintptr_t)buf % 16 == 0)
+        return fmt == 1 ? rows::launch_tile<float, HD>((float*)plane, pe, (float*)buf, which, r0, r1, dir, L)
+                        : rows::launch_tile<unsigned short, HD>((unsigned short*)plane, pe, (unsigned short*)buf, which, r0,
+                                                                r1, dir, L);
     if (fmt == 1)
         return dir == 0 ? launch(fl_rows<float, 0>, grid, dim3(256), L, (float*)plane, pe, (float*)buf, r0, r1, which)
                         : launch(fl_rows<float, 1>, grid, dim3(256), L, (float*)plane, pe, (float*)buf, r0, r1, which);

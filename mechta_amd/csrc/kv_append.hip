@@ -4,6 +4,7 @@
 // rope / rope2 / copy (ops.wgsl:141-162, 275-286) for the f32 cache. One launch writes K and V of all ntok tokens:
 // work items [0, nk) are K items (token, kv head, 8 dims), the rest V items (V group of positions, kv head, dim).
 #include "mkv_internal.h"
+#include "mkv_rows.h"
 
 namespace mkv {
 namespace {
@@ -70,7 +71,7 @@ __global__ void __launch_bounds__(256) append_kernel(void* __restrict__ kplane0,
 }
 
 // Position-major <-> store layout for [p0, p1) of one (layer, K|V): element (pos, kvh, d) of the reference layout
-// at ((pos - p0)*2 + kvh)*256 + d.
+// at ((pos - p0)*2 + kvh)*256 + d. For rows that are not 16-byte aligned; the others take rows_tile (mkv_rows.h).
 template <typename T, int DIR>  // DIR 0: store -> rows, 1: rows -> store
 __global__ void __launch_bounds__(256) rows_kernel(T* __restrict__ plane0, T* __restrict__ plane1,
                                                    T* __restrict__ rows, int p0, int p1, int which, int fmt) {
@@ -109,6 +110,10 @@ static hipError_t launch_rows(const Geom& g, const void* base, int layer, int wh
     void* q1 = b + g.plane(layer, which, 1) * g.plane_bytes();
     size_t total = (size_t)(p1 - p0) * KVH * HD;
     if (total == 0) return hipSuccess;
+    if ((uintptr_t)rows % 16 == 0)
+        return g.fmt == 0 ? rows::launch_tile<unsigned short, HD>((unsigned short*)q0, g.plane_elems, (unsigned short*)rows,
+                                                                  which, p0, p1, dir, L)
+                          : rows::launch_tile<float, HD>((float*)q0, g.plane_elems, (float*)rows, which, p0, p1, dir, L);
     unsigned blocks = (unsigned)((total + 255) / 256);
     if (g.fmt == 0)
         return launch(dir == 0 ? rows_kernel<unsigned short, 0> : rows_kernel<unsigned short, 1>, dim3(blocks),
