@@ -84,7 +84,7 @@ __global__ void __launch_bounds__(256) fl_attn(const void* __restrict__ kplane, 
     constexpr int BPE = FMT == 1 ? 4 : 2;
     constexpr unsigned TILE_BYTES = TILE * HD * BPE;
     const int G = gridDim.x, L = blockIdx.x;
-    const int W = G % NXCD == 0 ? (L % NXCD) * (G / NXCD) + L / NXCD : L;
+    const int W = xcd_order(L, G);
     const int rb = W % nrb, c = (W / nrb) % nch, kvh = W / nrb / nch;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, s = lane >> 5, r32 = lane & 31;
     const int t0 = 4 * rb, nt = min(4, T - t0);
@@ -316,7 +316,7 @@ __global__ void __launch_bounds__(PF_NW * 64) fl_pf(const void* __restrict__ kpl
     constexpr int SUB = Gm::SUB, TB = Gm::TILE_BYTES, SLOT = Gm::SLOT;
     // XCD-aware order (as the decode and prefill kernels): the token blocks of one (split, kv head) on one XCD
     const int G = gridDim.x, Lb = blockIdx.x;
-    const int W = G % NXCD == 0 ? (Lb % NXCD) * (G / NXCD) + Lb / NXCD : Lb;
+    const int W = xcd_order(Lb, G);
     const int nblk = (T + PF_PT - 1) / PF_PT;
     const int rb = W % nblk, c = (W / nblk) % nch, kvh = W / nblk / nch;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, r = lane & 31;

@@ -57,10 +57,9 @@ __global__ void __launch_bounds__(NTH, NWV == 4 ? 2 : 1) attn_f32(const float* _
                                                 float* __restrict__ part, const float* __restrict__ akn,
                                                 const float* __restrict__ av, const float* __restrict__ atab, int apos,
                                                 int antok) {
-    // XCD-aware order: consecutive work-groups go round robin to the 8 XCDs, so work item W = (L % 8) (G / 8) + L / 8
-    // puts the token blocks that stream the same keys on one XCD's L2
+    // XCD-aware order: the token blocks that stream the same keys on one XCD's L2
     const int G = gridDim.x, L = blockIdx.x;
-    const int W = G % NXCD == 0 ? (L % NXCD) * (G / NXCD) + L / NXCD : L;
+    const int W = xcd_order(L, G);
     const int ncg = nch - c0;
     const int rb = W % nrb, c = c0 + (W / nrb) % ncg, kvh = W / nrb / ncg;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, s = lane >> 5, r32 = lane & 31;

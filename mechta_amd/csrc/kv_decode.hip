@@ -61,13 +61,12 @@ __global__ void __launch_bounds__(512) decode_f16(_Float16* __restrict__ kplane,
                                                   const float* __restrict__ av, const float* __restrict__ atab,
                                                   int apos, int antok, int rpk, int cols) {
     // cols == 0: grid (splits, kv heads, token blocks). cols > 0 (small prefill blocks): a 1D grid of
-    // splits x kv heads x cols, ordered XCD-aware with the token blocks fastest: the dispatcher deals consecutive
-    // work-groups round robin to the 8 XCDs, so W = (L % 8) (G / 8) + L / 8 puts the cols work-groups that stream the
-    // same stage on one XCD, where all but the first find it in L2
+    // splits x kv heads x cols in XCD order with the token blocks fastest: the cols work-groups that stream the same stage
+    // are on one XCD, where all but the first find it in L2
     int kvh = blockIdx.y, c = blockIdx.x, nch = gridDim.x, zb = blockIdx.z;
     if (cols > 0) {
         const int G = gridDim.x, L = blockIdx.x;
-        const int W = G % NXCD == 0 ? (L % NXCD) * (G / NXCD) + L / NXCD : L;
+        const int W = xcd_order(L, G);
         nch = G / (KVH * cols);
         zb = W % cols;
         c = (W / cols) % nch;
@@ -630,6 +629,8 @@ hipError_t merge_as(const float* part, int rpk, int ntok, int n, int start, int 
     // block at 28,000 positions, 32 splits, 87.8 against 94.2 us per step; with 64 splits, four groups, slower than
     // decode_combine: 68.4 against 63.0 us)
     const dim3 few((ntok * QH + 3) / 4), rows(ntok * QH, HD / 64);
+    if (nch <= 4)
+        return launch(merge_few<false, H16, 4>, few, dim3(256), L, part, rpk, ntok, n, start, span, nch, gate, out);
     if (nch <= 8)  // the 8 splits of a 512-token block: 12.2 against 14.5 us with the 16-chunk build
         return launch(merge_few<false, H16, 8>, few, dim3(256), L, part, rpk, ntok, n, start, span, nch, gate, out);
     if (nch <= MERGE_FEW)

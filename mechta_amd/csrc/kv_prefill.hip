@@ -3,74 +3,71 @@
 // Replaces q_f16 + attn_fa_mx + attn_fd_combine of the reference's prefill (fa_mx.wgsl:19-115, 313-319;
 // engine.rs:1215-1236). Token t of the block (0-based) sees positions [start, n + t).
 //
-// Work-group = (32 tokens of the block, split of `ch` positions, kv head): 8 waves (two per SIMD, so one wave's
-// softmax overlaps the other's matrix work), each owns 4 tokens x the kv head's 8 query heads = 32 query rows
-// (row = token*8 + head). The split's 32-key tiles (a 16 KB K block and four 4 KB V groups, contiguous in HBM)
-// stream through a 4-slot LDS ring filled by direct global->LDS loads, shared by the 8 waves. Per tile and wave:
+// Work-group = (32 or 16 tokens of the block, key split, kv head): 8 waves (two per SIMD, so one wave's softmax overlaps
+// the other's matrix work), each owns 4 tokens x the kv head's 8 query heads = 32 query rows (row = token*8 + head) and,
+// with two key groups (PfGeom), every other tile. The split's 32-key tiles (a 16 KB K block and four 4 KB V groups,
+// contiguous in HBM) stream through an LDS ring filled by direct global->LDS loads, shared by the waves. Per tile and wave:
 //   S^T[32 keys][32 rows] = K . Q^T    16 x v_mfma_f32_32x32x16_f16 (A = K rows in key_perm order from LDS,
 //                                      B = Q rounded to f16, held in registers for the whole split)
 //   online softmax of the 32 rows in registers, lazy reference max (moves when first or when the tile max exceeds
 //   it by more than 8), row sums from the f32 P (as attn_fa_mx), P rounded to f16 for the matrix units
 //   O[32 rows][256] += P . V           16 x v_mfma_f32_32x32x16_f16 (A = P straight from the S registers,
 //                                      B = V from LDS)
-// Each wave writes one partial [m, l, acc[256]] per row; launch_merge combines the splits (and applies the gate).
+// One partial [m, l, acc[256]] per row; launch_merge combines the splits (and applies the gate).
+#include <type_traits>
+
 #include "mkv_device.h"
 
 namespace mkv {
 namespace {
 
-#ifndef MKV_PF_RB
-#define MKV_PF_RB 1
-#endif
-#ifndef MKV_PF_NW
-#define MKV_PF_NW 8
-#endif
-constexpr int RB = MKV_PF_RB;                 // 32-row blocks (4 tokens x 8 heads) per wave
-constexpr int NW = MKV_PF_NW;                 // waves per work-group
-constexpr int PT = NW * 4 * RB;               // tokens per work-group
-constexpr int SUB = 1;                        // 32-key subtiles per ring slot (per barrier)
+constexpr int NW = 8;                         // waves per work-group
 constexpr int TILE_BYTES = 32 * HD * 2;       // one 32-key K block (or its 4 V groups), f16
-constexpr int SLOT_BYTES = 2 * SUB * TILE_BYTES;  // K blocks, then V groups of a slot
-#ifndef MKV_PF_NSLOT
-#define MKV_PF_NSLOT 4
-#endif
-#ifndef MKV_PF_WGS_PER_CU
-#define MKV_PF_WGS_PER_CU 1
-#endif
-constexpr int NSLOT = MKV_PF_NSLOT;           // LDS ring slots: NSLOT - 1 tiles in flight while one is computed
-constexpr int WGS_PER_CU = MKV_PF_WGS_PER_CU;  // work-groups the plan places per CU
+constexpr int RING_BYTES = 8 * TILE_BYTES;    // LDS ring
 
-constexpr int LPT = 2 * SUB * TILE_BYTES / NW / 1024;  // direct loads per slot and wave
-static_assert(NSLOT == 2 || LPT == 4 || LPT == 8, "wait counts below");
+// KS: key groups of a work-group. KS = 1: its 8 waves hold 32 tokens and take every tile. KS = 2: waves 0-3 hold 16 tokens
+// and take the even tiles, waves 4-7 the same tokens and the odd tiles, and the two states of a row meet in LDS at the
+// end: half the split partials (and half of Q's reads) for the same work-groups, twice the tiles read from L2.
+template <int KS>
+struct PfGeom {
+    static constexpr int RW = NW / KS;                  // waves over the rows
+    static constexpr int PT = 4 * RW;                   // tokens per work-group
+    static constexpr int STEP_BYTES = 2 * KS * TILE_BYTES;  // K and V of a step's KS tiles
+    static constexpr int NSLOT = RING_BYTES / STEP_BYTES;   // ring slots: NSLOT - 1 steps in flight while one is computed
+    static constexpr int PART_BYTES = TILE_BYTES / RW;  // of its key group's K block (or V groups) a wave copies
+    static constexpr int LPT = 2 * PART_BYTES / 1024;   // direct loads per step and wave
+};
 
-__device__ inline void wait_tiles(int later) {  // at most `later` tiles (LPT direct loads each per wave) pending
-    if constexpr (NSLOT == 2) {
+template <int KS>
+__device__ inline void wait_steps(int later) {  // at most `later` steps (LPT direct loads each per wave) pending
+    if constexpr (KS == 2) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    } else if constexpr (LPT == 4) {
+    } else {
+        static_assert(PfGeom<1>::LPT == 4 && PfGeom<1>::NSLOT == 4, "wait counts");
         if (later >= 2) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
         else if (later == 1) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    } else {
-        if (later >= 2) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-        else if (later == 1) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
 }
 
+template <int KS>
 __global__ void __launch_bounds__(NW * 64) prefill_f16(const _Float16* __restrict__ kplane,
                                                    const _Float16* __restrict__ vplane, size_t plane_elems,
                                                    const float* __restrict__ q, int T, int n, int start, float scale2,
                                                    int span, int nch, float* __restrict__ part) {
-    // XCD-aware order: the dispatcher deals consecutive work-groups round robin to the 8 XCDs (each with its own
-    // L2), so work item W = xcd * (grid / 8) + slot keeps the token blocks of one (split, kv head) -- the
-    // work-groups that stream the same keys -- on one XCD, and each key is fetched into one L2 instead of eight.
+    // XCD-aware order with the token blocks of one (split, kv head) -- the work-groups that stream the same keys --
+    // neighbours: each key is fetched into one L2 instead of eight. For every grid: 200 tokens at 9,000 positions (252
+    // work-groups) took 66.2 us while only multiples of 8 were ordered, 62.7 since (one key group both times).
     const int G = gridDim.x, L = blockIdx.x;
-    const int W = G % NXCD == 0 ? (L % NXCD) * (G / NXCD) + L / NXCD : L;
+    const int W = xcd_order(L, G);
+    using Gm = PfGeom<KS>;
+    constexpr int PT = Gm::PT, PART_BYTES = Gm::PART_BYTES, NSLOT = Gm::NSLOT;
     const int nblk = (T + PT - 1) / PT;
     const int rb = W % nblk, sp = (W / nblk) % nch, kvh = W / nblk / nch, tid = threadIdx.x;
     const int lane = tid & 63, w = tid >> 6;
+    const int wr = w % Gm::RW, kg = __builtin_amdgcn_readfirstlane(w / Gm::RW);  // row wave, key group
     const int h = lane >> 5, r = lane & 31;
-    const int t0 = rb * PT + 4 * RB * w;     // this wave's first token; row block b holds tokens t0 + 4b .. +3
+    const int t0 = rb * PT + 4 * wr;         // this wave's first token
     const int tlast = min(T - 1, rb * PT + PT - 1);
     const int kend = n + T - 1;              // positions written for this block
     const int cs = chunk_lo(sp, span, nch), ce = min(sp + 1 < nch ? chunk_lo(sp + 1, span, nch) : span, n + tlast);
@@ -78,19 +75,20 @@ __global__ void __launch_bounds__(NW * 64) prefill_f16(const _Float16* __restric
     const _Float16* K = kplane + (size_t)kvh * plane_elems;
     const _Float16* V = vplane + (size_t)kvh * plane_elems;
 
-    __shared__ __attribute__((aligned(16))) unsigned char ring[NSLOT * SLOT_BYTES];
+    __shared__ __attribute__((aligned(16))) unsigned char ring[RING_BYTES];
     __shared__ __attribute__((aligned(16))) float cfs[NW][32];  // rescale factors of a wave's rows
-    const int ntiles = (ce - cs + 32 * SUB - 1) / (32 * SUB);
-    constexpr int PART_BYTES = SUB * TILE_BYTES / NW;
-    // the wave's part of a tile: a per-lane offset fixed for the kernel; the tile's base and LDS slot are wave-uniform
-    const unsigned voff = w * PART_BYTES + lane * 16;
-    const unsigned wlds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(lds_void*)ring + w * PART_BYTES);
-    // V rows past the written length may hold anything: each wave zeroes them in the part of tile j it copied itself,
+    const int ntiles = (ce - cs + 31) / 32, nsteps = (ntiles + KS - 1) / KS;
+    // step j is tiles KS j .. KS j + KS - 1; this wave copies a part of tile KS j + kg, the one it computes: a per-lane
+    // offset fixed for the kernel; the tile's base and LDS slot are wave-uniform
+    const unsigned voff = wr * PART_BYTES + lane * 16;
+    const unsigned wlds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(lds_void*)ring + kg * 2 * TILE_BYTES + wr * PART_BYTES);
+    auto kof = [&](int j) { return (j % NSLOT) * Gm::STEP_BYTES + kg * 2 * TILE_BYTES; };  // this key group's K of step j
+    // V rows past the written length may hold anything: each wave zeroes them in the part of the tile it copied itself,
     // after its own copies have landed and before the barrier that hands the tile to every wave (no barrier of its own)
     auto zero_own_tail = [&](int j) {
-        const int k0 = cs + 32 * SUB * j;
-        if (k0 + 32 * SUB <= kend) return;
-        unsigned char* Vw = ring + (j % NSLOT) * SLOT_BYTES + SUB * TILE_BYTES;
+        const int k0 = cs + 32 * (KS * j + kg);
+        if (k0 + 32 <= kend) return;
+        unsigned char* Vw = ring + kof(j) + TILE_BYTES;
 #pragma unroll
         for (int i = 0; i < PART_BYTES / 1024; i++) {
             const unsigned off = voff + i * 1024;  // 8 consecutive positions of one dim: group off / 4096
@@ -104,60 +102,63 @@ __global__ void __launch_bounds__(NW * 64) prefill_f16(const _Float16* __restric
             }
         }
     };
-    auto issue = [&](int j) {  // each wave copies 1/NW of tile j's K blocks and V groups into slot j % NSLOT
-        const int k0 = cs + 32 * SUB * j;
+    auto issue = [&](int j) {  // this wave's part of its tile's K block and V groups into slot j % NSLOT
+        const int k0 = cs + 32 * (KS * j + kg);
+        if (KS > 1 && KS * j + kg >= ntiles) return;
         const unsigned char* ks = (const unsigned char*)(K + (size_t)(k0 / KBLK) * (KBLK * HD));
         const unsigned char* vs = (const unsigned char*)(V + (size_t)(k0 / VGRP) * (VGRP * HD));
-        const unsigned dst = wlds + (j % NSLOT) * SLOT_BYTES;
+        const unsigned dst = wlds + (j % NSLOT) * Gm::STEP_BYTES;
 #pragma unroll
         for (int i = 0; i < PART_BYTES / 1024; i++) dma16s(ks + i * 1024, voff, dst + i * 1024);
 #pragma unroll
-        for (int i = 0; i < PART_BYTES / 1024; i++) dma16s(vs + i * 1024, voff, dst + SUB * TILE_BYTES + i * 1024);
+        for (int i = 0; i < PART_BYTES / 1024; i++) dma16s(vs + i * 1024, voff, dst + TILE_BYTES + i * 1024);
     };
-    for (int j = 0; j < NSLOT - 1 && j < ntiles; j++) issue(j);
+    for (int j = 0; j < NSLOT - 1 && j < nsteps; j++) issue(j);
 
-    // Q as the B operand of S^T: for row block b, lane (r, h) holds row r (token t0 + 4b + r/8, head r%8), dims
-    // 16s + 8h .. +7 for step s, rounded to f16 (q_f16); rows of tokens past the block are zero
-    half8 qb[RB][16];
-    int vis[RB];
-#pragma unroll
-    for (int b = 0; b < RB; b++) {
-        const int tr = t0 + 4 * b + (r >> 3);
-        vis[b] = tr < T ? n + tr : 0;  // row r of block b sees keys < vis[b]
+    // Q as the B operand of S^T: lane (r, h) holds row r (token t0 + r/8, head r%8), dims 16s + 8h .. +7 for step s, rounded
+    // to f16 (q_f16); rows of tokens past the block are zero
+    half8 qb[16];
+    const int tr = t0 + (r >> 3);
+    const int vis = tr < T ? n + tr : 0;  // row r sees keys < vis
+    {
         const float* qrow = q + ((size_t)min(tr, T - 1) * QH + kvh * GQA + (r & 7)) * HD + 8 * h;
 #pragma unroll
         for (int s = 0; s < 16; s++) {
             float4 x0 = *(const float4*)(qrow + 16 * s), x1 = *(const float4*)(qrow + 16 * s + 4);
             if (tr >= T) x0 = x1 = make_float4(0.f, 0.f, 0.f, 0.f);
-            qb[b][s] = half8{(_Float16)x0.x, (_Float16)x0.y, (_Float16)x0.z, (_Float16)x0.w,
-                             (_Float16)x1.x, (_Float16)x1.y, (_Float16)x1.z, (_Float16)x1.w};
+            qb[s] = half8{(_Float16)x0.x, (_Float16)x0.y, (_Float16)x0.z, (_Float16)x0.w,
+                          (_Float16)x1.x, (_Float16)x1.y, (_Float16)x1.z, (_Float16)x1.w};
         }
     }
     const int kaddr = h * 512 + key_perm(r) * 16;
-    // the smallest window end of each row block (its first token's; 0 when the block runs past T): a tile with every
-    // key below it, and none below start, needs no mask (a wave-uniform test)
-    int vmin[RB];
+    // the smallest window end of the wave's rows (its first token's; 0 when they run past T): a tile with every key below
+    // it, and none below start, needs no mask (a wave-uniform test)
+    const int tf = __builtin_amdgcn_readfirstlane(t0), vmin = tf + 3 < T ? n + tf : 0;
+    float m = NEG_INF, lsum = 0.f;
+    f32x16 O[8];
 #pragma unroll
-    for (int b = 0; b < RB; b++) {
-        const int tf = __builtin_amdgcn_readfirstlane(t0 + 4 * b);
-        vmin[b] = tf + 3 < T ? n + tf : 0;
-    }
-    float m[RB], lsum[RB];
-    f32x16 O[RB][8];
+    for (int nb = 0; nb < 8; nb++) O[nb] = f32x16{};
+    // O's rows times the factor of each, which lane (row) holds: register i of O holds row 8(i/4) + 4h + i%4, so the 32
+    // factors pass through this wave's LDS row (constant offsets, no per-register lane index to keep)
+    auto scale_rows = [&](float cf) {
+        if (h == 0) cfs[w][r] = cf;
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int b = 0; b < RB; b++) {
-        m[b] = NEG_INF;
-        lsum[b] = 0.f;
+        for (int a = 0; a < 4; a++) {
+            const f32x4 f = *(const f32x4*)&cfs[w][8 * a + 4 * h];
 #pragma unroll
-        for (int nb = 0; nb < 8; nb++) O[b][nb] = f32x16{};
-    }
+            for (int nb = 0; nb < 8; nb++) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) O[nb][4 * a + q] *= f[q];
+            }
+        }
+    };
 
-    // S of tile j, the mask where it crosses a row's window, the online softmax (lazy reference max, O rescaled when a
-    // finite reference moved) and P into pa
-    auto s_mfma = [&](int j, f32x16(&Scur)[RB]) {
-        const unsigned char* Ks = ring + (j % NSLOT) * SLOT_BYTES;
-#pragma unroll
-        for (int b = 0; b < RB; b++) Scur[b] = f32x16{};
+    // S of this wave's tile of step j, the mask where it crosses a row's window, the online softmax (lazy reference max, O
+    // rescaled when a finite reference moved) and P into pa
+    auto s_mfma = [&](int j, f32x16& S) {
+        const unsigned char* Ks = ring + kof(j);
+        S = f32x16{};
         constexpr int KP = 3;  // K operands in flight ahead of the S chain (LDS latency; 4 to 6 measured no faster)
         half8 kbuf[KP];
 #pragma unroll
@@ -166,8 +167,7 @@ __global__ void __launch_bounds__(NW * 64) prefill_f16(const _Float16* __restric
         for (int s = 0; s < 16; s++) {
             const half8 ka = kbuf[s % KP];
             if (s + KP < 16) kbuf[s % KP] = *(const half8*)(Ks + kaddr + (s + KP) * 1024);
-#pragma unroll
-            for (int b = 0; b < RB; b++) Scur[b] = mfma32(ka, qb[b][s], Scur[b]);
+            S = mfma32(ka, qb[s], S);
         }
         // schedule: KP LDS reads (mask 0x100), then alternately one MFMA (0x008) and the next LDS read
         __builtin_amdgcn_sched_group_barrier(0x100, KP, 0);
@@ -178,64 +178,49 @@ __global__ void __launch_bounds__(NW * 64) prefill_f16(const _Float16* __restric
         }
         __builtin_amdgcn_sched_group_barrier(0x008, KP, 0);
     };
-    auto softmax = [&](int j, f32x16(&Scur)[RB], half8(&pa)[RB][2]) {
-        const int k0 = cs + 32 * j;
-#pragma unroll
-        for (int b = 0; b < RB; b++) {
-            // the causal / start mask only where this tile crosses a row's window (raw scores; the scale, log2
-            // units, is applied to the max and inside the exponent's FMA)
-            if (!(k0 >= start && k0 + 32 <= vmin[b])) {
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const int key = k0 + 8 * h + i + (i >= 8 ? 8 : 0);
-                    Scur[b][i] = (key < vis[b] && key >= start) ? Scur[b][i] : NEG_INF;
-                }
-            }
-            // the first maximum is the compiler's: it reads the MFMA results and so carries the wait states a
-            // vector read of them needs, which inline assembly would not get; the rest follows it
-            float mt = fmaxf(Scur[b][0], Scur[b][1]);
-#pragma unroll
-            for (int i = 2; i < 16; i += 2) mt = vmax3(mt, Scur[b][i], Scur[b][i + 1]);
-            mt = max_xor32(mt);
-            mt *= scale2;  // scale2 > 0: the max of the scaled scores is the scaled max
-            // the reference max moves when first or when the tile max exceeds it by more than 8; O and the sum are
-            // rescaled only when a finite reference moved (rare: the exponential is not evaluated otherwise)
-            const bool rescale = m[b] != NEG_INF && mt > m[b] + LAZY2;
-            const float mr = m[b] == NEG_INF || rescale ? fmaxf(m[b], mt) : m[b];
-            float cf = 1.f;
-            if (__any(rescale)) {
-                // register i of O holds row 8(i/4) + 4h + i%4, whose factor lane (that row) holds: the 32 factors pass
-                // through this wave's LDS row (constant offsets, no per-register lane index to keep)
-                cf = rescale ? fast_exp2(m[b] - mr) : 1.f;
-                if (h == 0) cfs[w][r] = cf;
-                __builtin_amdgcn_wave_barrier();
-#pragma unroll
-                for (int a = 0; a < 4; a++) {
-                    const f32x4 f = *(const f32x4*)&cfs[w][8 * a + 4 * h];
-#pragma unroll
-                    for (int nb = 0; nb < 8; nb++) {
-#pragma unroll
-                        for (int q = 0; q < 4; q++) O[b][nb][4 * a + q] *= f[q];
-                    }
-                }
-            }
-            m[b] = mr;
-            // P = 2^(s * scale2 - m) (one FMA): masked scores are -inf and give 0 (the reference is 0 while a row has seen no key);
-            // the row sum takes the f32 P, as attn_fa_mx does, the P.V operand its f16 rounding
-            const float base = mr == NEG_INF ? 0.f : mr;
-            float ls;
+    auto softmax = [&](int j, f32x16& S, half8(&pa)[2]) {
+        const int k0 = cs + 32 * (KS * j + kg);
+        // the causal / start mask only where this tile crosses a row's window (raw scores; the scale, log2 units, is
+        // applied to the max and inside the exponent's FMA)
+        if (!(k0 >= start && k0 + 32 <= vmin)) {
 #pragma unroll
             for (int i = 0; i < 16; i++) {
-                const float p = fast_exp2(__builtin_fmaf(Scur[b][i], scale2, -base));
-                ls = i == 0 ? p : ls + p;  // 0 + p0 is p0: the same sum without the first add
-                pa[b][i >> 3][i & 7] = (_Float16)p;
+                const int key = k0 + 8 * h + i + (i >= 8 ? 8 : 0);
+                S[i] = (key < vis && key >= start) ? S[i] : NEG_INF;
             }
-            lsum[b] = lsum[b] * cf + ls;
         }
+        // the first maximum is the compiler's: it reads the MFMA results and so carries the wait states a vector read of
+        // them needs, which inline assembly would not get; the rest follows it
+        float mt = fmaxf(S[0], S[1]);
+#pragma unroll
+        for (int i = 2; i < 16; i += 2) mt = vmax3(mt, S[i], S[i + 1]);
+        mt = max_xor32(mt);
+        mt *= scale2;  // scale2 > 0: the max of the scaled scores is the scaled max
+        // the reference max moves when first or when the tile max exceeds it by more than 8; O and the sum are rescaled
+        // only when a finite reference moved (rare: the exponential is not evaluated otherwise)
+        const bool rescale = m != NEG_INF && mt > m + LAZY2;
+        const float mr = m == NEG_INF || rescale ? fmaxf(m, mt) : m;
+        float cf = 1.f;
+        if (__any(rescale)) {
+            cf = rescale ? fast_exp2(m - mr) : 1.f;
+            scale_rows(cf);
+        }
+        m = mr;
+        // P = 2^(s * scale2 - m) (one FMA): masked scores are -inf and give 0 (the reference is 0 while a row has seen no
+        // key); the row sum takes the f32 P, as attn_fa_mx does, the P.V operand its f16 rounding
+        const float base = mr == NEG_INF ? 0.f : mr;
+        float ls;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const float p = fast_exp2(__builtin_fmaf(S[i], scale2, -base));
+            ls = i == 0 ? p : ls + p;  // 0 + p0 is p0: the same sum without the first add
+            pa[i >> 3][i & 7] = (_Float16)p;
+        }
+        lsum = lsum * cf + ls;
     };
-    // O += P . V of tile j
-    auto pv_tile = [&](int j, const half8(&pa)[RB][2]) {
-        const unsigned char* Vs = ring + (j % NSLOT) * SLOT_BYTES + TILE_BYTES;
+    // O += P . V of this wave's tile of step j
+    auto pv_tile = [&](int j, const half8(&pa)[2]) {
+        const unsigned char* Vs = ring + kof(j) + TILE_BYTES;
         constexpr int VP = 3;  // V operands in flight ahead of the P.V MFMAs
         half8 vbuf[VP];
         auto vaddr = [&](int i) { return Vs + (2 * (i >> 3) + h) * 4096 + (32 * (i & 7) + r) * 16; };
@@ -245,8 +230,7 @@ __global__ void __launch_bounds__(NW * 64) prefill_f16(const _Float16* __restric
         for (int i = 0; i < 16; i++) {
             const half8 vb = vbuf[i % VP];
             if (i + VP < 16) vbuf[i % VP] = *(const half8*)vaddr(i + VP);
-#pragma unroll
-            for (int b = 0; b < RB; b++) O[b][i & 7] = mfma32(pa[b][i >> 3], vb, O[b][i & 7]);
+            O[i & 7] = mfma32(pa[i >> 3], vb, O[i & 7]);
         }
         __builtin_amdgcn_sched_group_barrier(0x100, VP, 0);
 #pragma unroll
@@ -256,38 +240,85 @@ __global__ void __launch_bounds__(NW * 64) prefill_f16(const _Float16* __restric
         }
         __builtin_amdgcn_sched_group_barrier(0x008, VP, 0);
     };
-    for (int j = 0; j < ntiles; j++) {
-        wait_tiles(min(ntiles - 1 - j, NSLOT - 2));
+    for (int j = 0; j < nsteps; j++) {
+        wait_steps<KS>(min(nsteps - 1 - j, NSLOT - 2));
         zero_own_tail(j);
-        lds_barrier();  // tile j is in LDS for every wave; every wave is done with tile j - 1
-        if (j + NSLOT - 1 < ntiles) issue(j + NSLOT - 1);  // into the slot of tile j - 1
-        f32x16 S[RB];
-        half8 pa[RB][2];
+        lds_barrier();  // step j is in LDS for every wave; every wave is done with step j - 1
+        if (j + NSLOT - 1 < nsteps) issue(j + NSLOT - 1);  // into the slot of step j - 1
+        if (KS > 1 && KS * j + kg >= ntiles) break;        // no odd tile in the last step
+        f32x16 S;
+        half8 pa[2];
         s_mfma(j, S);
         softmax(j, S, pa);
         pv_tile(j, pa);
     }
+    lsum += __shfl_xor(lsum, 32);
 
     // partials of this wave's rows of present tokens: row index t*8 + head of the kv head, rows per kv head = 8T
     const size_t rpk = (size_t)T * GQA;
-#pragma unroll
-    for (int b = 0; b < RB; b++) {
-        lsum[b] += __shfl_xor(lsum[b], 32);
-        const int tb = t0 + 4 * b;
+    auto row_part = [&](int ri) { return part + ((kvh * rpk + (size_t)t0 * GQA + ri) * nch + sp) * PART; };
+    auto store_o = [&](auto nb0, auto cnt) {  // dim blocks nb0 .. nb0 + cnt - 1 of O
 #pragma unroll
         for (int i = 0; i < 16; i++) {
             const int ri = 8 * (i >> 2) + 4 * h + (i & 3);
-            if (tb + (ri >> 3) < T) {
-                float* p = part + ((kvh * rpk + (size_t)tb * GQA + ri) * nch + sp) * PART + PACC + r;
+            if (t0 + (ri >> 3) < T) {
+                float* p = row_part(ri) + PACC + r;
 #pragma unroll
-                for (int nb = 0; nb < 8; nb++) p[32 * nb] = O[b][nb][i];
+                for (int nb = 0; nb < cnt; nb++) p[32 * (nb0 + nb)] = O[nb0 + nb][i];
             }
         }
-        if (h == 0 && tb + (r >> 3) < T) {
-            float* p = part + ((kvh * rpk + (size_t)tb * GQA + r) * nch + sp) * PART;
-            p[0] = m[b];
-            p[1] = lsum[b];
+    };
+    using std::integral_constant;
+    if constexpr (KS == 1) {
+        store_o(integral_constant<int, 0>{}, integral_constant<int, 8>{});
+    } else {
+        // the row's two states, waves w and w ^ 4: both scaled to the common maximum, each wave then takes over half of the
+        // dims (its partner's half of them through the ring, which no wave reads any more behind the first barrier)
+        __shared__ __attribute__((aligned(16))) float ml[NW][2][32];
+        if (h == 0) {
+            ml[w][0][r] = m;
+            ml[w][1][r] = lsum;
         }
+        __syncthreads();
+        const float mo = ml[w ^ Gm::RW][0][r], lo = ml[w ^ Gm::RW][1][r];
+        const float M = fmaxf(m, mo);
+        const float f = m == NEG_INF ? 0.f : fast_exp2(m - M), fo = mo == NEG_INF ? 0.f : fast_exp2(mo - M);
+        scale_rows(f);
+        f32x4* const mine = (f32x4*)ring + w * 1024 + lane;
+        const f32x4* const other = (const f32x4*)ring + (w ^ Gm::RW) * 1024 + lane;
+        auto give = [&](auto nb0) {
+#pragma unroll
+            for (int nb = 0; nb < 4; nb++)
+#pragma unroll
+                for (int a = 0; a < 4; a++)
+                    mine[(nb * 4 + a) * 64] = f32x4{O[nb0 + nb][4 * a], O[nb0 + nb][4 * a + 1], O[nb0 + nb][4 * a + 2],
+                                                    O[nb0 + nb][4 * a + 3]};
+        };
+        auto take = [&](auto nb0) {
+#pragma unroll
+            for (int nb = 0; nb < 4; nb++)
+#pragma unroll
+                for (int a = 0; a < 4; a++) {
+                    const f32x4 x = other[(nb * 4 + a) * 64];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) O[nb0 + nb][4 * a + e] += x[e];
+                }
+            store_o(nb0, integral_constant<int, 4>{});
+        };
+        const integral_constant<int, 0> low{};
+        const integral_constant<int, 4> high{};
+        if (kg == 0) give(high);
+        else give(low);
+        __syncthreads();
+        if (kg == 0) take(low);
+        else take(high);
+        m = M;
+        lsum = lsum * f + lo * fo;
+    }
+    if (kg == 0 && h == 0 && t0 + (r >> 3) < T) {
+        float* p = row_part(r);
+        p[0] = m;
+        p[1] = lsum;
     }
 }
 
@@ -316,7 +347,7 @@ __global__ void __launch_bounds__(P32_NW * 64) prefill_f32(const float* __restri
                                                           const float* __restrict__ q, int T, int n, int start,
                                                           float scale2, int span, int nch, float* __restrict__ part) {
     const int G = gridDim.x, Lb = blockIdx.x;
-    const int W = G % NXCD == 0 ? (Lb % NXCD) * (G / NXCD) + Lb / NXCD : Lb;
+    const int W = xcd_order(Lb, G);
     const int nblk = (T + P32_PT - 1) / P32_PT;
     const int rb = W % nblk, sp = (W / nblk) % nch, kvh = W / nblk / nch, tid = threadIdx.x;
     const int lane = tid & 63, w = tid >> 6, h = lane >> 5, r = lane & 31, blk = w >> 1, dh = w & 1;
@@ -522,14 +553,23 @@ __global__ void __launch_bounds__(P32_NW * 64) prefill_f32(const float* __restri
 // at most 16, a 64-token block at 28,000 positions took 95 us on 64 work-groups, now 64 us on 256 (f32 store: 16
 // tokens 197 -> 65 us). The workspace bound, tokens x splits <= 4,096, is unchanged.
 constexpr int PF_MAXCH = 64;
-PrefillPlan prefill_plan(int T, int n) {
-    const int kend = n + T - 1;
-    const int blocks = 2 * ((T + PT - 1) / PT);  // work-groups per split
-    int nch = 256 * WGS_PER_CU / blocks;         // about WGS_PER_CU work-groups per CU
-    const int most = kend / 64;                  // splits of at least 64 positions
+static int prefill_splits(int T, int kend, int pt) {
+    int nch = 256 / (2 * ((T + pt - 1) / pt));  // about one work-group per CU
+    const int most = kend / 64;                 // splits of at least 64 positions
     nch = nch > most ? most : nch;
-    nch = nch < 1 ? 1 : nch > PF_MAXCH ? PF_MAXCH : nch;
-    return PrefillPlan{kend, nch};
+    return nch < 1 ? 1 : nch > PF_MAXCH ? PF_MAXCH : nch;
+}
+
+PrefillPlan prefill_plan(int T, int n) {
+    // One or two key groups per work-group: a call takes about 32.5 us + 1.72 us per tile of a wave with one and 25.5 us +
+    // 1.85 us with two (512 tokens at 1,000 / 4,000 / 9,000 / 16,000 / 28,000 positions, with the merge and the gate: 42.4
+    // / 62.1 / 94.8 / 141 / 224 against 36.2 / 57.2 / 93.1 / 144 / 245 us), so two groups serve up to about 50 tiles per
+    // wave. Blocks of 16 tokens instead of 32 also round ragged blocks less: 200 tokens at 9,000 positions 62.7 against
+    // 52.5 us.
+    const int kend = n + T - 1;
+    const int nch1 = prefill_splits(T, kend, PfGeom<1>::PT), nch2 = prefill_splits(T, kend, PfGeom<2>::PT);
+    const int s1 = kend / (32 * nch1), s2 = kend / (64 * nch2);  // tiles per wave
+    return 700 + 172 * s1 > 185 * s2 ? PrefillPlan{kend, nch2, 2} : PrefillPlan{kend, nch1, 1};
 }
 
 PrefillPlan prefill32_plan(int T, int n) {
@@ -539,7 +579,7 @@ PrefillPlan prefill32_plan(int T, int n) {
     const int most = kend / 64;                           // splits of at least 64 positions
     nch = nch > most ? most : nch;
     nch = nch < 1 ? 1 : nch > PF_MAXCH ? PF_MAXCH : nch;
-    return PrefillPlan{kend, nch};
+    return PrefillPlan{kend, nch, 1};
 }
 
 size_t prefill_ws_floats(int T, int nch) { return (size_t)KVH * T * GQA * nch * PART; }
@@ -550,9 +590,9 @@ hipError_t launch_prefill(const Geom& g, const void* base, int layer, const floa
     const char* b = (const char*)base;
     const void* kp = b + g.plane(layer, 0, 0) * g.plane_bytes();
     const void* vp = b + g.plane(layer, 1, 0) * g.plane_bytes();
-    dim3 grid((T + PT - 1) / PT * p.nch * KVH);
-    return launch(prefill_f16, grid, dim3(NW * 64), L, kp, vp, g.plane_elems, q, T, n, start, scale * LOG2E, p.span,
-                  p.nch, ws);
+    const int pt = p.ks == 2 ? PfGeom<2>::PT : PfGeom<1>::PT;
+    return launch(p.ks == 2 ? prefill_f16<2> : prefill_f16<1>, dim3((T + pt - 1) / pt * p.nch * KVH), dim3(NW * 64), L, kp,
+                  vp, g.plane_elems, q, T, n, start, scale * LOG2E, p.span, p.nch, ws);
 }
 
 hipError_t launch_prefill_f32(const Geom& g, const void* base, int layer, const float* q, int T, int n, int start,

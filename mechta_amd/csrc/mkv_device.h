@@ -15,6 +15,14 @@ constexpr float LOG2E = 1.4426950408889634f;
 constexpr float LAZY2 = 8.0f * LOG2E;  // DM_LAZY = 8 (dmx.rs:124) in log2 units
 constexpr float NEG_INF = -__builtin_huge_valf();
 
+// Work item of work-group L of a 1D grid of G: the dispatcher deals consecutive work-groups round robin to the 8 XCDs
+// (each with its own L2), so XCD L % 8 takes a contiguous range of the items, and the items that stream the same keys,
+// being neighbours, share an L2. Any G: the first G % 8 XCDs take one item more.
+__device__ inline int xcd_order(int L, int G) {
+    const int x = L % NXCD, q = G / NXCD, e = G % NXCD;
+    return x * q + (x < e ? x : e) + L / NXCD;
+}
+
 // 2^x with the hardware's v_exp_f32 (no denormal scaffolding: results below 2^-126 flush to 0, far below the
 // smallest f16 P of 2^-24).
 __device__ inline float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }

@@ -183,6 +183,7 @@ hipError_t launch_attn_f32(const Geom& g, const void* base, int layer, const flo
 // Prefill: split-K pass into the partials ws, then launch_merge with the returned plan.
 struct PrefillPlan {
     int span, nch;  // splits of [0, span) as chunk_lo
+    int ks;         // f16: key groups per work-group (1 or 2)
 };
 PrefillPlan prefill_plan(int T, int n);
 size_t prefill_ws_floats(int T, int nch);
