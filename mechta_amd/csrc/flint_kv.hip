@@ -367,16 +367,9 @@ __global__ void __launch_bounds__(PF_NW * 64) fl_pf(const void* __restrict__ kpl
     // into f16 hi + lo; rows of tokens past the block are zero and see no key
     const int tr = tb + 4 * w + (r >> 3);
     const int vlo = tr < T ? window_lo(pos0 + tr, win) : 0, vhi = tr < T ? pos0 + tr + 1 : 0;  // row sees [vlo, vhi)
-    half8 qh[8], ql[8];
-    {
-        const float* qrow = q + ((size_t)min(tr, T - 1) * QH + kvh * GQA + (r & 7)) * HD + 8 * h;
-#pragma unroll
-        for (int s = 0; s < 8; s++) {
-            f32x4 x0 = *(const f32x4*)(qrow + 16 * s), x1 = *(const f32x4*)(qrow + 16 * s + 4);
-            if (tr >= T) x0 = x1 = f32x4{};
-            split8(x0, x1, qh[s], ql[s]);
-        }
-    }
+    half8 qh[8], ql[8];  // through the ring's last slot, which no load fills before the first slot's barrier
+    static_assert(SLOT >= PF_NW * 4096, "4 KB per wave");
+    stage_q32(q + (size_t)kvh * GQA * HD, QH * HD, HD, T, tb + 4 * w, lane, ring + (PF_NSLOT - 1) * SLOT + w * 4096, qh, ql);
     // K in a tile: f16 [dims/8][32 keys][8], f32 [dims/4][32 keys][4]; lane (r, h) of step s takes dims 16s + 8h .. +7
     // of key key_perm(r)
     const int kaddr = FMT == 1 ? h * 1024 + key_perm(r) * 16 : h * 512 + key_perm(r) * 16;

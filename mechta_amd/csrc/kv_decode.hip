@@ -600,16 +600,29 @@ SmallPlan small_prefill_plan(int T, int n, int start) {
     DecodePlan d = decode_plan(n, T, start);
     const int kend = n + T - 1, nu = (kend - d.s0 + KPS_F16 - 1) / KPS_F16;
     d.nch = min(max(nu, 1), SMALL_WG);
-    const int cap = max(8, SMALL_WG / nzb);  // twice or four times as many splits measured slower
+    // twice or four times as many splits measured slower; larger blocks (small_prefill_pays): one work-group per CU
+    const int cap = T <= SMALL_PREFILL_MAX ? max(8, SMALL_WG / nzb) : max(1, 128 / nzb);
     d.nch = min(d.nch, cap);
     return SmallPlan{d, nzb};
+}
+
+bool small_prefill_pays(int T, int n, int start) {
+    // about 10.3 us + 1.25 us per stage of a work-group, against the model of prefill_plan. Per call, on this path against
+    // prefill_f16: 64 tokens at 300 / 1,000 / 4,000 / 9,000 positions 11.6 / 13.9 / 21.1 / 32.8 against 17.4 / 19.0 / 26.2 /
+    // 31.5 us, 128 tokens at 300 / 1,000 / 4,000 13.4 / 17.6 / 32.1 against 18.0 / 21.7 / 31.0, 256 tokens at 300 / 1,000
+    // 18.5 / 24.4 against 21.8 / 26.2 us
+    if (T > 256) return false;  // no faster there (512 tokens at 300 positions 31 against 27-29 us)
+    const SmallPlan p = small_prefill_plan(T, n, start);
+    int other;
+    (void)prefill_plan(T, n, &other);
+    return 1030 + 125 * ((p.d.nu + p.d.nch - 1) / p.d.nch) < other;
 }
 
 size_t small_prefill_ws_floats(int T, int nch) { return (size_t)KVH * 32 * ((T + 3) / 4) * nch * PART; }
 
 hipError_t launch_small_prefill(const Geom& g, const void* base, int layer, const float* q, int T, int n, int start,
                                 float scale, const SmallPlan& p, float* ws, const Launch& L) {
-    if (g.fmt != 0 || T < 1 || T > SMALL_PREFILL_MAX) return hipErrorNotSupported;
+    if (g.fmt != 0 || T < 1) return hipErrorNotSupported;
     char* b = (char*)base;
     void* kp = b + g.plane(layer, 0, 0) * g.plane_bytes();
     void* vp = b + g.plane(layer, 1, 0) * g.plane_bytes();

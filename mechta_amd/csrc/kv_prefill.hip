@@ -14,6 +14,7 @@
 //   O[32 rows][256] += P . V           16 x v_mfma_f32_32x32x16_f16 (A = P straight from the S registers,
 //                                      B = V from LDS)
 // One partial [m, l, acc[256]] per row; launch_merge combines the splits (and applies the gate).
+#include <climits>
 #include <type_traits>
 
 #include "mkv_device.h"
@@ -120,16 +121,9 @@ __global__ void __launch_bounds__(NW * 64) prefill_f16(const _Float16* __restric
     half8 qb[16];
     const int tr = t0 + (r >> 3);
     const int vis = tr < T ? n + tr : 0;  // row r sees keys < vis
-    {
-        const float* qrow = q + ((size_t)min(tr, T - 1) * QH + kvh * GQA + (r & 7)) * HD + 8 * h;
-#pragma unroll
-        for (int s = 0; s < 16; s++) {
-            float4 x0 = *(const float4*)(qrow + 16 * s), x1 = *(const float4*)(qrow + 16 * s + 4);
-            if (tr >= T) x0 = x1 = make_float4(0.f, 0.f, 0.f, 0.f);
-            qb[s] = half8{(_Float16)x0.x, (_Float16)x0.y, (_Float16)x0.z, (_Float16)x0.w,
-                          (_Float16)x1.x, (_Float16)x1.y, (_Float16)x1.z, (_Float16)x1.w};
-        }
-    }
+    // through the ring's last slot, which no load fills before the first tile's barrier
+    stage_q16(q + (size_t)kvh * GQA * HD, QH * HD, HD, T, t0, lane, ring + (NSLOT - 1) * Gm::STEP_BYTES + w * 4096, qb);
+    __builtin_amdgcn_sched_barrier(0);  // the loads' registers are free before O takes its own
     const int kaddr = h * 512 + key_perm(r) * 16;
     // the smallest window end of the wave's rows (its first token's; 0 when they run past T): a tile with every key below
     // it, and none below start, needs no mask (a wave-uniform test)
@@ -388,16 +382,8 @@ __global__ void __launch_bounds__(P32_NW * 64) prefill_f32(const float* __restri
     // Q: lane (r, h) holds row r (token t0 + r / 8, head r % 8), dims 128dh + 16s + 8h .. +7 of step s, split
     const int tr = t0 + (r >> 3);
     const int vis = tr < T ? n + tr : 0;  // row r sees keys [start, vis)
-    half8 qh[8], ql[8];
-    {
-        const float* qrow = q + ((size_t)min(tr, T - 1) * QH + kvh * GQA + (r & 7)) * HD + 128 * dh + 8 * h;
-#pragma unroll
-        for (int s = 0; s < 8; s++) {
-            f32x4 x0 = *(const f32x4*)(qrow + 16 * s), x1 = *(const f32x4*)(qrow + 16 * s + 4);
-            if (tr >= T) x0 = x1 = f32x4{};
-            split8(x0, x1, qh[s], ql[s]);
-        }
-    }
+    half8 qh[8], ql[8];  // through the ring's second slot, which no load fills before the first tile's barrier
+    stage_q32(q + (size_t)kvh * GQA * HD + 128 * dh, QH * HD, HD, T, t0, lane, ring + P32_SLOT + w * 4096, qh, ql);
     const int kaddr = (32 * dh + 2 * h) * 512 + key_perm(r) * 16;  // K chunk (dims / 4) 32dh + 4s + 2h, +1
     float m = NEG_INF, lsum = 0.f;
     f32x16 O[4];
@@ -553,23 +539,37 @@ __global__ void __launch_bounds__(P32_NW * 64) prefill_f32(const float* __restri
 // at most 16, a 64-token block at 28,000 positions took 95 us on 64 work-groups, now 64 us on 256 (f32 store: 16
 // tokens 197 -> 65 us). The workspace bound, tokens x splits <= 4,096, is unchanged.
 constexpr int PF_MAXCH = 64;
-static int prefill_splits(int T, int kend, int pt) {
-    int nch = 256 / (2 * ((T + pt - 1) / pt));  // about one work-group per CU
-    const int most = kend / 64;                 // splits of at least 64 positions
-    nch = nch > most ? most : nch;
-    return nch < 1 ? 1 : nch > PF_MAXCH ? PF_MAXCH : nch;
+// The cheapest split count of one work-group shape by a model of the call (0.01 us): what does not depend on the splits,
+// a wave's tiles, and what each split adds to the merge and in partials written and read back.
+static PrefillPlan best_splits(int T, int kend, int pt, int ks, int& cost) {
+    const int blocks = 2 * ((T + pt - 1) / pt), tiles = (kend + 31) / 32;
+    int most = 256 / blocks;  // at most about one work-group per CU
+    most = most > PF_MAXCH ? PF_MAXCH : most < 1 ? 1 : most;
+    PrefillPlan p{kend, 1, ks};
+    cost = INT_MAX;
+    for (int nch = 1; nch <= most && (nch == 1 || nch * ks <= tiles); nch++) {
+        const int s = (tiles + nch * ks - 1) / (nch * ks);  // tiles of a wave
+        const int t = ks == 1 ? 1100 + 135 * s : 1230 + 145 * s + (s > 40 ? 50 * (s - 40) : 0);
+        const int c = t + nch * T * 55 / 100 + 20 * nch;
+        if (c < cost) {
+            cost = c;
+            p.nch = nch;
+        }
+    }
+    return p;
 }
 
-PrefillPlan prefill_plan(int T, int n) {
-    // One or two key groups per work-group: a call takes about 32.5 us + 1.72 us per tile of a wave with one and 25.5 us +
-    // 1.85 us with two (512 tokens at 1,000 / 4,000 / 9,000 / 16,000 / 28,000 positions, with the merge and the gate: 42.4
-    // / 62.1 / 94.8 / 141 / 224 against 36.2 / 57.2 / 93.1 / 144 / 245 us), so two groups serve up to about 50 tiles per
-    // wave. Blocks of 16 tokens instead of 32 also round ragged blocks less: 200 tokens at 9,000 positions 62.7 against
-    // 52.5 us.
+PrefillPlan prefill_plan(int T, int n, int* us100) {
+    // Measured per call with merge and gate. 512 tokens at 1,000 / 4,000 / 9,000 / 16,000 / 28,000 positions: one key group
+    // 42.4 / 62.1 / 94.8 / 141 / 224, two 36.2 / 57.2 / 93.1 / 144 / 245 us: two groups read each tile for half as many rows
+    // (which tells on long splits, where the card is power limited) and save half the partials. Splits, two groups: 64
+    // tokens at 4,000 positions on 32 / 16 / 8 splits 32.7 / 26.4 / 26.2, at 9,000 34.4 / 31.5 / 38.7, 128 tokens at 2,000
+    // on 16 / 8 32.5 / 26.0 us.
     const int kend = n + T - 1;
-    const int nch1 = prefill_splits(T, kend, PfGeom<1>::PT), nch2 = prefill_splits(T, kend, PfGeom<2>::PT);
-    const int s1 = kend / (32 * nch1), s2 = kend / (64 * nch2);  // tiles per wave
-    return 700 + 172 * s1 > 185 * s2 ? PrefillPlan{kend, nch2, 2} : PrefillPlan{kend, nch1, 1};
+    int c1, c2;
+    const PrefillPlan p1 = best_splits(T, kend, PfGeom<1>::PT, 1, c1), p2 = best_splits(T, kend, PfGeom<2>::PT, 2, c2);
+    if (us100) *us100 = c2 <= c1 ? c2 : c1;
+    return c2 <= c1 ? p2 : p1;
 }
 
 PrefillPlan prefill32_plan(int T, int n) {

@@ -130,19 +130,10 @@ hipError_t decode_all(mkv_store* h, const DecodeWs& ws, int layer, const float* 
                   [&](const Launch& L) { return launch_decode_merge(ntok, n, start, p, ws, gate, out, h16, L); });
 }
 
-// Floats of the prefill partials workspace, allocated with the store: the largest any prefill plan uses (the f16
-// plans keep T * splits <= 4096, the f32 plan <= 2048, the small-block plan <= 4096 rows per kv head).
-size_t prefill_ws_max_floats() {
-    size_t m = 0;
-    for (int T = 1; T <= MKV_PREFILL_MAX; T++) {
-        for (int n : {1, 64, 1024, 8192, MKV_CTX_MAX - T}) {
-            m = std::max(m, prefill_ws_floats(T, prefill_plan(T, n).nch));
-            m = std::max(m, prefill_ws_floats(T, prefill32_plan(T, n).nch));
-            if (T <= SMALL_PREFILL_MAX) m = std::max(m, small_prefill_ws_floats(T, small_prefill_plan(T, n, 0).d.nch));
-        }
-    }
-    return m;
-}
+// Floats of the prefill partials workspace, allocated with the store: the f16 and f32 plans keep tokens x splits <= 4,096
+// (256 work-groups of 32 tokens over both kv heads), the small-block plans <= 4,096 rows x splits per kv head; mkv_prefill
+// checks every call's plan against it.
+constexpr size_t PREFILL_WS_FLOATS = (size_t)KVH * 4096 * GQA * PART;
 
 void free_events(mkv_store* h) {
     for (auto& s : h->pending) {
@@ -156,7 +147,7 @@ void free_events(mkv_store* h) {
 
 // Device bytes of one store: the planes (layers x {K, V} x 2 heads x ctx x 256 elements: exactly the reference's
 // 2 x layers KV buffers of buffer_bytes_for(ctx), engine.rs:64-65) plus the slack past the last plane, then the decode
-// partials (2 kv heads x 32 rows x splits x 260 floats) and the prefill partials (prefill_ws_max_floats).
+// partials (2 kv heads x 32 rows x splits x 260 floats) and the prefill partials (PREFILL_WS_FLOATS).
 struct StoreBytes {
     size_t planes, slack, decode_ws, prefill_ws;
     int max_chunks;
@@ -169,7 +160,7 @@ StoreBytes store_bytes(int layers, int ctx, int fmt) {
     // decode splits: f16 one per 64-position stage, at most 108 (small prefill blocks 124); f32 at most 248
     b.max_chunks = std::min(ctx / 64 + 2, 256);
     b.decode_ws = (size_t)KVH * ROWS * b.max_chunks * PART * sizeof(float);
-    b.prefill_ws = prefill_ws_max_floats() * sizeof(float);
+    b.prefill_ws = PREFILL_WS_FLOATS * sizeof(float);
     return b;
 }
 
@@ -434,8 +425,8 @@ int mkv_prefill(mkv_t* h, int layer, const float* q, int T, int n, int start, fl
     if (int rc = check_attn(h, "mkv_prefill", layer, q, T, MKV_PREFILL_MAX, n, start, out)) return rc;
     hipError_t e = hipSuccess;
     int span = 0, nch = 0, rpk = T * GQA;  // the split-K plan the merge reads
-    if (h->g.fmt == MKV_F16 && T <= SMALL_PREFILL_MAX) {
-        // blocks under 64 tokens: f32-class, as the reference's attn_fd4 (engine.rs:1237-1241)
+    if (h->g.fmt == MKV_F16 && (T <= SMALL_PREFILL_MAX || small_prefill_pays(T, n, start))) {
+        // blocks under 64 tokens: f32-class, as the reference's attn_fd4 (engine.rs:1237-1241); larger ones where it is faster
         const SmallPlan p = small_prefill_plan(T, n, start);
         if (small_prefill_ws_floats(T, p.d.nch) > h->pws_floats) return fail(MKV_E_ARG, "mkv_prefill: workspace");
         span = p.d.span;

@@ -136,6 +136,76 @@ __device__ inline half8 bload16(rsrc_t r, unsigned off) {
     return __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, LOAD_NT));
 }
 
+// The Q operands of a prefill wave: 32 rows (row = token * 8 + head of tokens t0 .. t0 + 3; rows of tokens past T are zero),
+// NS steps of 16 dims; lane (r, h) gets row r, dims 16s + 8h .. +7 of step s. q: dim 0 of the kv head's first row of token
+// 0, tokens tstride and heads hstride floats apart. Loaded as the matrix units want it, each load instruction would touch
+// 32 rows in 16-byte pieces (a 64-token block at 300 positions took 19.8 us, most of it that); here a load takes whole
+// 256-byte (16 steps' f16: 4 rows) or 128-byte (split: 8 rows) runs, all of them in flight at once, and the operands turn
+// in 4 KB of the wave's own LDS, 64 (f16) or 32 (split) dims a round. A row's round is 8 chunks of 16 bytes, chunk c of
+// row r at c ^ (r & 7): reads of 32 rows hit every bank.
+template <int NS>
+__device__ inline void stage_q16(const float* __restrict__ q, int tstride, int hstride, int T, int t0, int lane,
+                                 unsigned char* lds, half8 (&qb)[NS]) {
+    constexpr int RND = NS / 4;
+    const int sub = lane & 15, rr = lane >> 4, r = lane & 31, h = lane >> 5;
+    f32x4 x[RND][8];
+#pragma unroll
+    for (int k = 0; k < RND; k++)
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int row = 4 * i + rr, t = t0 + (row >> 3);
+            x[k][i] = *(const f32x4*)(q + (size_t)min(t, T - 1) * tstride + (row & 7) * hstride + 64 * k + 4 * sub);
+        }
+#pragma unroll
+    for (int k = 0; k < RND; k++) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int row = 4 * i + rr;
+            const f32x4 y = t0 + (row >> 3) < T ? x[k][i] : f32x4{};
+            *(half4*)(lds + row * 128 + (((sub >> 1) ^ (row & 7)) * 16) + (sub & 1) * 8) =
+                half4{(_Float16)y.x, (_Float16)y.y, (_Float16)y.z, (_Float16)y.w};
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int s = 0; s < 4; s++) qb[4 * k + s] = *(const half8*)(lds + r * 128 + (((2 * s + h) ^ (r & 7)) * 16));
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+template <int NS>
+__device__ inline void stage_q32(const float* __restrict__ q, int tstride, int hstride, int T, int t0, int lane,
+                                 unsigned char* lds, half8 (&qh)[NS], half8 (&ql)[NS]) {
+    constexpr int RND = NS / 2;
+    const int sub = lane & 7, rr = lane >> 3, r = lane & 31, h = lane >> 5;
+    f32x4 x[RND][4];
+#pragma unroll
+    for (int k = 0; k < RND; k++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int row = 8 * i + rr, t = t0 + (row >> 3);
+            x[k][i] = *(const f32x4*)(q + (size_t)min(t, T - 1) * tstride + (row & 7) * hstride + 32 * k + 4 * sub);
+        }
+#pragma unroll
+    for (int k = 0; k < RND; k++) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int row = 8 * i + rr;
+            const f32x4 y = t0 + (row >> 3) < T ? x[k][i] : f32x4{};
+            half4 hi, lo;
+            split4(y, hi, lo);
+            unsigned char* p = lds + row * 128 + (sub & 1) * 8;
+            *(half4*)(p + (((sub >> 1) ^ (row & 7)) * 16)) = hi;
+            *(half4*)(p + (((4 + (sub >> 1)) ^ (row & 7)) * 16)) = lo;
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            qh[2 * k + s] = *(const half8*)(lds + r * 128 + (((2 * s + h) ^ (r & 7)) * 16));
+            ql[2 * k + s] = *(const half8*)(lds + r * 128 + (((4 + 2 * s + h) ^ (r & 7)) * 16));
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
 // Work-group barrier for LDS traffic only: waits for this wave's LDS operations, not for its global loads (a
 // __syncthreads() would also wait for every pending global load and drain the loads already in flight).
 __device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }

@@ -150,15 +150,17 @@ hipError_t launch_decode_core(const Geom& g, void* base, int layer, const float*
                               const Launch& L);
 hipError_t launch_decode_merge(int ntok, int n, int start, const DecodePlan& p, const DecodeWs& ws, const float* gate,
                                void* out, bool h16, const Launch& L);
-// Small prefill blocks on the f16 store (T < SMALL_PREFILL_MAX): the reference runs them through attn_fd4 (f32 Q,
-// exact f32 softmax; engine.rs:1237-1241), so they run on decode_f16's f32-class arithmetic, one column of work-groups
-// per block of 4 tokens over the decode's stages; partials [kvh][row < 32 nzb][nch][PART], then launch_merge.
+// Small prefill blocks on the f16 store (T <= SMALL_PREFILL_MAX): the reference runs them through attn_fd4 (f32 Q, exact
+// f32 softmax; engine.rs:1237-1241), so they run on decode_f16's f32-class arithmetic, one column of work-groups per block
+// of 4 tokens over the decode's stages; partials [kvh][row < 32 nzb][nch][PART], then launch_merge. Larger blocks take the
+// same kernel where the context is short (small_prefill_pays): it has little to set up.
 constexpr int SMALL_PREFILL_MAX = 63;
 struct SmallPlan {
     DecodePlan d;
     int nzb;  // blocks of 4 tokens
 };
 SmallPlan small_prefill_plan(int T, int n, int start);
+bool small_prefill_pays(int T, int n, int start);  // T > SMALL_PREFILL_MAX: faster there than on prefill_f16
 size_t small_prefill_ws_floats(int T, int nch);
 hipError_t launch_small_prefill(const Geom& g, const void* base, int layer, const float* q, int T, int n, int start,
                                 float scale, const SmallPlan& p, float* ws, const Launch& L);
@@ -185,7 +187,7 @@ struct PrefillPlan {
     int span, nch;  // splits of [0, span) as chunk_lo
     int ks;         // f16: key groups per work-group (1 or 2)
 };
-PrefillPlan prefill_plan(int T, int n);
+PrefillPlan prefill_plan(int T, int n, int* us100 = nullptr);  // us100: the plan's modelled time (0.01 us)
 size_t prefill_ws_floats(int T, int nch);
 hipError_t launch_prefill(const Geom& g, const void* base, int layer, const float* q, int T, int n, int start,
                           float scale, const PrefillPlan& p, float* ws, const Launch& L);
