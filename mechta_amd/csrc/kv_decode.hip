@@ -640,7 +640,8 @@ hipError_t merge_as(const float* part, int rpk, int ntok, int n, int start, int 
     if (nch > 16 * MERGE_JMAX) return hipErrorInvalidValue;
     // few chunks, or many rows (prefill blocks) over up to two groups of chunks: a row per 64 threads (a 128-token
     // block at 28,000 positions, 32 splits, 87.8 against 94.2 us per step; with 64 splits, four groups, slower than
-    // decode_combine: 68.4 against 63.0 us)
+    // decode_combine: 68.4 against 63.0 us); with few rows decode_combine's smaller work-groups are faster (32 tokens of
+    // the f32 store at 4,000 positions, 32 splits: 30.8 against 34.3 us)
     const dim3 few((ntok * QH + 3) / 4), rows(ntok * QH, HD / 64);
     if (nch <= 4)
         return launch(merge_few<false, H16, 4>, few, dim3(256), L, part, rpk, ntok, n, start, span, nch, gate, out);
@@ -649,7 +650,7 @@ hipError_t merge_as(const float* part, int rpk, int ntok, int n, int start, int 
     if (nch <= MERGE_FEW)
         return launch(merge_few<false, H16, MERGE_FEW>, few, dim3(256), L, part, rpk, ntok, n, start, span, nch, gate,
                       out);
-    if (ntok >= 32 && nch <= 2 * MERGE_FEW)
+    if (ntok >= 64 && nch <= 2 * MERGE_FEW)
         return launch(merge_few<true, H16, MERGE_FEW>, few, dim3(256), L, part, rpk, ntok, n, start, span, nch, gate,
                       out);
     if (nch <= 16 * 9)

@@ -535,9 +535,8 @@ __global__ void __launch_bounds__(P32_NW * 64) prefill_f32(const float* __restri
 
 }  // namespace
 
-// Splits per prefill plan at most: about one work-group per CU down to blocks of 64 tokens (f16) or 5 (f32); with
-// at most 16, a 64-token block at 28,000 positions took 95 us on 64 work-groups, now 64 us on 256 (f32 store: 16
-// tokens 197 -> 65 us). The workspace bound, tokens x splits <= 4,096, is unchanged.
+// Splits per f16 plan at most: about one work-group per CU down to blocks of 64 tokens; with at most 16, a 64-token block
+// at 28,000 positions took 95 us on 64 work-groups, 64 us on 256. The workspace bound is tokens x splits <= 4,096.
 constexpr int PF_MAXCH = 64;
 // The cheapest split count of one work-group shape by a model of the call (0.01 us): what does not depend on the splits,
 // a wave's tiles, and what each split adds to the merge and in partials written and read back.
@@ -573,12 +572,21 @@ PrefillPlan prefill_plan(int T, int n, int* us100) {
 }
 
 PrefillPlan prefill32_plan(int T, int n) {
-    const int kend = n + T - 1;
-    const int blocks = KVH * ((T + P32_PT - 1) / P32_PT);  // work-groups per split
-    int nch = 256 / blocks;                               // about one work-group per CU
-    const int most = kend / 64;                           // splits of at least 64 positions
-    nch = nch > most ? most : nch;
-    nch = nch < 1 ? 1 : nch > PF_MAXCH ? PF_MAXCH : nch;
+    // As best_splits (0.01 us): 2.55 us per tile of a work-group against the partials and the merge, whose kernel for more
+    // than 16 splits takes about 3 us longer. 5 tokens at 1,000 / 9,000 / 20,000 positions 17.9 / 27.6 / 44.5 us on at most
+    // 64 splits of at least 64 positions, 14.4 / 21.7 / 32.7 on these; 64 tokens at 1,000 positions on 8 / 16 / 32 splits
+    // 26.1 / 24.6 / 31.4, at 4,000 59.5 / 41.6 / 38.4 us.
+    const int kend = n + T - 1, tiles = (kend + 31) / 32;
+    int most = 256 / (KVH * ((T + P32_PT - 1) / P32_PT));  // at most about one work-group per CU
+    most = most < 1 ? 1 : most;
+    int best = INT_MAX, nch = 1;
+    for (int k = 1; k <= most && k <= tiles; k++) {
+        const int c = 255 * tiles / k + (T < 64 ? k * T * 45 / 100 : k * T * 55 / 100 + 8 * k) + (k > 16 ? 300 : 0);
+        if (c < best) {
+            best = c;
+            nch = k;
+        }
+    }
     return PrefillPlan{kend, nch, 1};
 }
 
