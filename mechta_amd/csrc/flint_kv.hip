@@ -1002,8 +1002,10 @@ __global__ void __launch_bounds__(256) fl_dec16(const void* __restrict__ kplane,
 // splits of a row loaded in one round trip.
 constexpr int MERGE_FEW = 16;
 
+// four work-groups per CU: without the bound the 8-split build took 218 registers (two waves per SIMD; 256 tokens of a
+// sliding layer 30.5 against 27.6 us per call)
 template <int NJ>  // at most NJ splits
-__global__ void __launch_bounds__(256) fl_merge_few(const float* __restrict__ part, int T, int nch,
+__global__ void __launch_bounds__(256, 4) fl_merge_few(const float* __restrict__ part, int T, int nch,
                                                     const float* __restrict__ sinks, float* __restrict__ out) {
     const int rowid = blockIdx.x * 8 + (threadIdx.x >> 5);  // t * 32 + head
     if (rowid >= T * QH) return;
@@ -1055,12 +1057,29 @@ Plan plan(int fmt, int pos0, int T, int win) {
     } else if (T <= 4) {  // one block of fl_attn: splits of at least 128 positions, 64 per kv head at most
         nch = span / 128;
         nch = nch > 64 ? 64 : nch;
-    } else {  // fl_pf: blocks of 32 tokens, about one work-group per CU, splits of 64 positions or more, at most 64
+    } else {
+        // fl_pf: blocks of 32 tokens, at most about one work-group per CU; the splits by a model of the call (0.01 us): a
+        // block's tiles against what each split adds in partials and merge, whose kernel for more than 16 splits takes
+        // longer on many rows. f32 cache, us per call on splits of at least 64 positions for every CU / on these: 5 tokens
+        // at 100 / 2,000 / 20,000 positions 17.5 / 16.7 / 38.2 -> 12.1 / 13.7 / 36.9, 64 tokens at 600 / 2,000 20.4 / 29.6 ->
+        // 19.6 / 26.9, 256 tokens at 600 34.1 -> 28.4, of a sliding layer 31.7 -> 26.1.
         nrb = (T + PF_PT - 1) / PF_PT;
-        nch = 256 / (nrb * KVH);
-        const int most = span / 64, room = WS_ROWS / (T * GQA);
-        nch = nch > most ? most : nch;
-        nch = nch > room ? room : nch > 64 ? 64 : nch;
+        const int blk = T < PF_PT ? T : PF_PT;
+        const int keys = win > 0 && win + blk - 1 < span ? win + blk - 1 : span;  // of one block
+        const int tiles = (keys + 31) / 32, tile = fmt == 1 ? 220 : 140;
+        const int per = T * 7 / 10 < 80 + T / 4 ? T * 7 / 10 : 80 + T / 4;
+        int most = 256 / (nrb * KVH);
+        const int room = WS_ROWS / (T * GQA);
+        most = most > room ? room : most > 64 ? 64 : most;
+        long best = -1;
+        nch = 1;
+        for (int k = 1; k <= most && k <= tiles; k++) {
+            const long c = (long)tile * ((tiles + k - 1) / k) + per * k + (k > 16 && T >= 32 ? 150 : 0);
+            if (best < 0 || c < best) {
+                best = c;
+                nch = k;
+            }
+        }
     }
     nch = nch < 1 ? 1 : nch;
     return Plan{klo, span, nch, nrb, fused};
