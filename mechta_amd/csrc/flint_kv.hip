@@ -1,9 +1,10 @@
 // flint_kv.hip -- the Flint model's KV path: ring append, NEOX RoPE, conversion to the reference's row layout, and
 // sliding-window attention with per-head sinks (flint_attn.wgsl:1-257), for one decode token or a prefill block.
 //
-// Three attention kernels: fl_dec16 (1-2 tokens, 16 query rows), fl_attn (3-4 tokens) and fl_pf (prefill blocks of
-// 5-512 tokens, 32 tokens per work-group sharing an LDS ring of K/V tiles). fl_attn's work-group: (block of 4 tokens,
-// key split, kv head) = 32 query rows (token * 8 + head) against the split's keys in tiles of 32 positions. The
+// Three attention kernels: fl_dec16 (1-2 tokens over long spans, 16 query rows), fl_attn (1-4 tokens, larger blocks over
+// short spans) and fl_pf (blocks of 5-512 tokens, 32 per work-group sharing an LDS ring of K/V tiles). fl_attn's
+// work-group: (block of 4 tokens, key split, kv head) = 32 query rows (token * 8 + head) against the split's keys in
+// tiles of 32 positions. The
 // arithmetic is f32, as the reference's, taken on the f16 matrix units: f32 operands are split into f16 hi + lo and
 // each product is three v_mfma_f32_32x32x16_f16 passes (hi.hi + hi.lo + lo.hi, f32 accumulation), two where one side
 // is an f16 cache's K or V (exact in f16). Per tile, wave w of 4:
@@ -35,24 +36,17 @@ namespace {
 #define FL_DEC_NCH 48     // decode: splits per kv head at most (32,768 positions: 48 against 32 / 64 / 96 splits
                           // 17.9-18.3 against 19.2 / 18.3-18.5 / 19.7 us per f16 call)
 #endif
-#ifndef FL_FUSE_NCH
-#define FL_FUSE_NCH 8     // decode with the merge fused (short spans): splits per kv head at most
+// Decodes (1-2 tokens) of more than these many positions take fl_dec16, whose waves keep more of the keys in flight;
+// shorter ones fl_attn, whose splits of one tile finish sooner. One token on a full layer, us per call, on fl_dec16 (up
+// to 384 positions f32 and 512 f16 with the merge in the kernel) / fl_attn: f32 at 100 / 544 / 1,200 / 2,040 / 3,060
+// positions 8.6 / 9.4 / 9.9 / 10.5 / 11.0 -> 7.1 / 8.0 / 8.2 / 8.4 / 9.8, f16 up to 2,040 7.9 / 8.4 / 8.8 / 9.1 -> 7.0 /
+// 7.1 / 7.5 / 7.9; a sliding layer 9.7 -> 7.9 and 8.8 -> 7.5. Past the line (three tokens on fl_attn against one on
+// fl_dec16): f32 at 5,000 12.6 against 11.7, f16 at 2,500 9.9 against 9.4.
+#ifndef FL_DEC_SPAN_F32
+#define FL_DEC_SPAN_F32 3072
 #endif
-#ifndef FL_FUSE_SPLIT
-#define FL_FUSE_SPLIT 80  // decode with the merge fused: positions per split at least (at 544 positions: 6 splits;
-                          // against 8 / 7 / 5 / 4 splits 9.8 against 10.7 / 9.8 / 10.0 / 10.7 us per f32 call, 8.6
-                          // against 8.8 / 8.6 / 8.5 / 8.8 us per f16 call)
-#endif
-// Decodes of spans up to these many positions merge in the kernel; longer ones launch the merge. One token on a full
-// layer, us per call with the merge in the kernel against two launches: f32 at 320 / 384 / 448 / 512 / 768 / 2,048
-// positions 9.1 / 9.5 / 10.1 / 10.2 / 10.4 / 13.0 against 9.0 / 9.5 / 9.8 / 9.9 / 9.6 / 10.7; f16 8.1 / 8.3 / 8.6 / 8.8
-// / 9.0 / 10.4 against 8.2 / 8.6 / 8.8 / 9.0 / 8.7 / 9.2; at 256 positions 9.0 / 8.2 against 10.7 / 10.2 (f32 / f16).
-// A sliding layer's 513-544 positions: 9.8 / 8.6 against 8.9 / 8.3.
-#ifndef FL_FUSE_SPAN_F32
-#define FL_FUSE_SPAN_F32 384
-#endif
-#ifndef FL_FUSE_SPAN_F16
-#define FL_FUSE_SPAN_F16 512
+#ifndef FL_DEC_SPAN_F16
+#define FL_DEC_SPAN_F16 2048
 #endif
 
 constexpr int TILE = 32;
@@ -728,8 +722,7 @@ template <int FMT, int NBUF>
 __global__ void __launch_bounds__(256) fl_dec16(const void* __restrict__ kplane, const void* __restrict__ vplane,
                                                 size_t plane_elems, int rows, const float* __restrict__ q, int T,
                                                 int pos0, int win, float scale2, int klo, int span, int nch,
-                                                float* __restrict__ part, unsigned* __restrict__ arrivals,
-                                                const float* __restrict__ sinks, float* __restrict__ out) {
+                                                float* __restrict__ part) {
     constexpr int BPE = FMT == 1 ? 4 : 2;
     const int c = blockIdx.x % nch, kvh = blockIdx.x / nch;
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, r16 = lane & 15;
@@ -892,13 +885,6 @@ __global__ void __launch_bounds__(256) fl_dec16(const void* __restrict__ kplane,
         ml[w][1][r16] = l_run;
     }
     __syncthreads();
-    // With the merge fused (arrivals != NULL, few splits), the partial is stored device-coherent (scope bit sc1,
-    // through the XCD's L2) and the kv head's last work-group to arrive merges them all; no work-group waits.
-    const bool fused = arrivals != nullptr;
-    auto put = [&](float* p, float x) {
-        if (fused) __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        else *p = x;
-    };
     const size_t rbase = (size_t)kvh * T * GQA;
     {
         // every wave combines dims 16cc .. 16cc + 15 of cc = 2w, 2w + 1 for its lane's rows 4g + r: the rows' factors
@@ -928,7 +914,7 @@ __global__ void __launch_bounds__(256) fl_dec16(const void* __restrict__ kplane,
                     float o = 0.f;
 #pragma unroll
                     for (int ww = 0; ww < 4; ww++) o += f[ww][r] * x[c2][ww][r];
-                    put(p + 16 * (2 * w + c2), o);
+                    p[16 * (2 * w + c2)] = o;
                 }
             }
         }
@@ -941,61 +927,9 @@ __global__ void __launch_bounds__(256) fl_dec16(const void* __restrict__ kplane,
         for (int ww = 0; ww < 4; ww++)
             Lt += ml[ww][0][r16] == NEG_INF ? 0.f : exp2f(ml[ww][0][r16] - M) * ml[ww][1][r16];
         float* p = part + ((rbase + r16) * nch + c) * PART;
-        put(p, M);
-        put(p + 1, Lt);
+        p[0] = M;
+        p[1] = Lt;
     }
-    if (!fused) return;
-    // every wave's partial stores complete before the work-group barrier; wave 0 then releases at agent scope: the
-    // partial happens before the arrival that counts it, and the kv head's last arrival acquires, so its merge reads
-    // every partial
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    __shared__ int last;
-    if (w == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        int l = 0;
-        if (lane == 0) {
-            l = __hip_atomic_fetch_add(arrivals + kvh, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                (unsigned)(nch - 1);
-            if (l) __hip_atomic_store(arrivals + kvh, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            last = l;
-        }
-        if (__builtin_amdgcn_readfirstlane(l)) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    }
-    __syncthreads();  // the other waves see the acquiring wave's view through the work-group barrier
-    if (!last) return;
-    // the kv head's last work-group: the merge of fl_merge for its rows (row = token * 8 + head of the kv head, T * 8
-    // <= 16), thread = (row, 8 dims), every split's partial loaded in one round trip (device-coherent loads)
-    const int row = tid >> 4, d0 = (tid & 15) * 8;
-    if (row >= T * GQA) return;
-    const int head = kvh * GQA + (row & 7), t = row >> 3;
-    const rsrc_t pr = plane_rsrc(part + (size_t)kvh * T * GQA * nch * PART, (unsigned)(T * GQA * nch * PART * 4));
-    f32x4 hd[FL_FUSE_NCH], a0[FL_FUSE_NCH], a1[FL_FUSE_NCH];
-#pragma unroll
-    for (int cj = 0; cj < FL_FUSE_NCH; cj++) {
-        const unsigned off = cj < nch ? (unsigned)(((row * nch + cj) * PART) * 4) : 0x7FFFFFF0u;
-        const unsigned oa = off + (PACC + d0) * 4;
-        hd[cj] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(pr, off, 0, LOAD_SC1));
-        a0[cj] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(pr, oa, 0, LOAD_SC1));
-        a1[cj] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(pr, oa + 16, 0, LOAD_SC1));
-    }
-    const float sk = sinks ? sinks[head] * LOG2E : NEG_INF;
-    float M = sk;
-#pragma unroll
-    for (int cj = 0; cj < FL_FUSE_NCH; cj++)
-        if (cj < nch) M = fmaxf(M, hd[cj].x);
-    f32x4 s0 = f32x4{}, s1 = f32x4{};
-    float L = sinks && M != NEG_INF ? exp2f(sk - M) : 0.f;
-#pragma unroll
-    for (int cj = 0; cj < FL_FUSE_NCH; cj++) {
-        const float e = cj < nch && hd[cj].x != NEG_INF ? exp2f(hd[cj].x - M) : 0.f;
-        L += e * hd[cj].y;
-        s0 += e * a0[cj];
-        s1 += e * a1[cj];
-    }
-    float* o = out + ((size_t)t * QH + head) * HD + d0;
-    *(f32x4*)o = s0 / L;
-    *(f32x4*)(o + 4) = s1 / L;
 }
 
 // Merge for few splits (prefill blocks): 8 rows (token, head) per work-group of 256 threads, 4 dims per thread, the
@@ -1042,50 +976,60 @@ __global__ void __launch_bounds__(256, 4) fl_merge_few(const float* __restrict__
 
 Plan plan(int fmt, int pos0, int T, int win) {
     const int lo0 = win > 0 && pos0 + 1 > win ? pos0 + 1 - win : 0;
-    const int klo = lo0 / 32 * 32, span = pos0 + T - klo;
+    const int klo = lo0 / 32 * 32;
+    int span = pos0 + T - klo;
     int nrb = (T + 3) / 4;
-    int nch;
-    int fused = 0;
-    if (T <= 2 && span <= (fmt == 1 ? FL_FUSE_SPAN_F32 : FL_FUSE_SPAN_F16)) {  // fl_dec16 merging its own partials:
-                                                                              // splits of at least FL_FUSE_SPLIT
-        nch = span / FL_FUSE_SPLIT;
-        nch = nch > FL_FUSE_NCH ? FL_FUSE_NCH : nch;
-        fused = 1;
-    } else if (T <= 2) {  // fl_dec16
+    int nch, blk = 4;
+    if (T <= 2 && span > (fmt == 1 ? FL_DEC_SPAN_F32 : FL_DEC_SPAN_F16)) {  // fl_dec16
+        blk = T;
         nch = span / FL_DEC_SPLIT;
         nch = nch > FL_DEC_NCH ? FL_DEC_NCH : nch;
-    } else if (T <= 4) {  // one block of fl_attn: splits of at least 128 positions, 64 per kv head at most
-        nch = span / 128;
-        nch = nch > 64 ? 64 : nch;
     } else {
-        // fl_pf: blocks of 32 tokens, at most about one work-group per CU; the splits by a model of the call (0.01 us): a
-        // block's tiles against what each split adds in partials and merge, whose kernel for more than 16 splits takes
-        // longer on many rows. f32 cache, us per call on splits of at least 64 positions for every CU / on these: 5 tokens
-        // at 100 / 2,000 / 20,000 positions 17.5 / 16.7 / 38.2 -> 12.1 / 13.7 / 36.9, 64 tokens at 600 / 2,000 20.4 / 29.6 ->
-        // 19.6 / 26.9, 256 tokens at 600 34.1 -> 28.4, of a sliding layer 31.7 -> 26.1.
-        nrb = (T + PF_PT - 1) / PF_PT;
-        const int blk = T < PF_PT ? T : PF_PT;
-        const int keys = win > 0 && win + blk - 1 < span ? win + blk - 1 : span;  // of one block
-        const int tiles = (keys + 31) / 32, tile = fmt == 1 ? 220 : 140;
-        const int per = T * 7 / 10 < 80 + T / 4 ? T * 7 / 10 : 80 + T / 4;
-        int most = 256 / (nrb * KVH);
-        const int room = WS_ROWS / (T * GQA);
-        most = most > room ? room : most > 64 ? 64 : most;
+        // 3 tokens and more, and short spans: kernel and splits with the least modelled time (0.01 us), tiles per split
+        // against what each split adds in partials and merge. fl_pf (32-token blocks, at most about one work-group per
+        // CU; a block's splits divide its own keys; merges of more than 16 splits take longer on many rows) or fl_attn
+        // (4-token blocks: every block reads the keys again, and work-groups on one CU share its rate, but a work-group
+        // starts 2 us sooner). Measured, f32 cache, us per call:
+        // - fl_attn, splits of 128 positions and more / by the model: 4 tokens at 200 / 600 / 2,500 / 5,000 positions
+        //   16.2 / 14.1 / 14.4 / 14.8 -> 7.9 / 8.7 / 10.9 / 13.0
+        // - fl_pf, splits of 64 positions and more for every CU / by the model / fl_attn: 5 tokens at 100 / 600 / 2,500
+        //   positions 17.7 / 16.3 / 18.1, 12.1 / 12.3 / 16.3, 7.9 / 8.7 / 12.0; 64 tokens at 300 19.4, 17.0, 12.6.
+        // - fl_pf: 64 tokens at 2,000 29.6 -> 26.9, 256 tokens at 600 34.1 -> 28.4, of a sliding
+        //   layer 31.7 -> 26.1.
+        const int per = T * 7 / 10 < 80 + T / 4 ? T * 7 / 10 : 80 + T / 4;  // per split
+        const int room = WS_ROWS / (T * GQA), cap = room < 64 ? room : 64;
         long best = -1;
         nch = 1;
-        for (int k = 1; k <= most && k <= tiles; k++) {
-            const long c = (long)tile * ((tiles + k - 1) / k) + per * k + (k > 16 && T >= 32 ? 150 : 0);
+        const int whole = (span + TILE - 1) / TILE, abase = fmt == 1 ? 850 : 830;
+        for (int k = 1; k <= cap && k <= whole; k++) {
+            const int percu = (nrb * KVH * k + 255) / 256;  // work-groups
+            const int tile = percu == 1 ? (fmt == 1 ? 135 : 120) : percu * (fmt == 1 ? 95 : 85);
+            const long c = abase + (long)tile * ((whole + k - 1) / k) + per * k;
             if (best < 0 || c < best) {
                 best = c;
                 nch = k;
             }
         }
+        const int prb = (T + PF_PT - 1) / PF_PT, pblk = T < PF_PT ? T : PF_PT;
+        const int keys = win > 0 && win + pblk - 1 < span ? win + pblk - 1 : span;  // of one block
+        const int tiles = (keys + TILE - 1) / TILE, tile = fmt == 1 ? 220 : 140, base = fmt == 1 ? 1050 : 950;
+        const int most = 256 / (prb * KVH) < cap ? 256 / (prb * KVH) : cap;
+        for (int k = 1; T > 4 && (k == 1 || (k <= most && k <= tiles)); k++) {
+            const long c = base + (long)tile * ((tiles + k - 1) / k) + per * k + (k > 16 && T >= 32 ? 150 : 0);
+            if (best < 0 || c < best) {
+                best = c;
+                nch = k;
+                blk = PF_PT;
+                nrb = prb;
+            }
+        }
+        if (blk == 4) span = (span + TILE - 1) / TILE * TILE;  // whole tiles divide evenly
     }
     nch = nch < 1 ? 1 : nch;
-    return Plan{klo, span, nch, nrb, fused};
+    return Plan{klo, span, nch, nrb, blk};
 }
 
-size_t ws_floats() { return (size_t)KVH * WS_ROWS * PART + WS_ARRIVALS; }
+size_t ws_floats() { return (size_t)KVH * WS_ROWS * PART; }
 
 hipError_t launch_attn(int fmt, const void* kp, const void* vp, int rows, const float* q, int T, int pos0, int win,
                        const Plan& p, float* ws, const float* sinks, float* out, hipStream_t st) {
@@ -1095,16 +1039,12 @@ hipError_t launch_attn(int fmt, const void* kp, const void* vp, int rows, const 
     const dim3 grid(p.nrb * p.nch * KVH);
     const Launch L{st};
     hipError_t e;
-    // arrival counters of the fused decode merge, zero between launches, after the partials
-    unsigned* arr = p.fused ? (unsigned*)(ws + (size_t)KVH * WS_ROWS * PART) : nullptr;
-    if (p.fused && p.nch > FL_FUSE_NCH) return hipErrorInvalidValue;
-    if (T <= 2) {  // decode (and 2-token steps): 16-row kernel
+    if (p.blk <= 2) {  // decode (and 2-token steps): 16-row kernel
         e = fmt == 1 ? launch(fl_dec16<1, FL_DEC_BUF>, dim3(p.nch * KVH), dim3(256), L, kp, vp, pe, rows, q, T, pos0,
-                              win, scale2, p.klo, p.span, p.nch, ws, arr, sinks, out)
+                              win, scale2, p.klo, p.span, p.nch, ws)
                      : launch(fl_dec16<0, FL_DEC_BUF>, dim3(p.nch * KVH), dim3(256), L, kp, vp, pe, rows, q, T, pos0,
-                              win, scale2, p.klo, p.span, p.nch, ws, arr, sinks, out);
-        if (p.fused) return e;
-    } else if (T <= 4) {  // one block of 4 tokens
+                              win, scale2, p.klo, p.span, p.nch, ws);
+    } else if (p.blk == 4) {  // blocks of 4 tokens
         e = fmt == 1 ? launch(fl_attn<1, 2>, grid, dim3(256), L, kp, vp, pe, rows, q, T, pos0, win, scale2, p.klo,
                               p.span, p.nch, p.nrb, ws)
                      : launch(fl_attn<0, 2>, grid, dim3(256), L, kp, vp, pe, rows, q, T, pos0, win, scale2, p.klo,

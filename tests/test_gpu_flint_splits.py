@@ -1,4 +1,4 @@
-"""Flint blocks (fl_pf, 5 tokens and more) at the edges of their split plan: splits of one tile, a last split of a few
+"""Flint blocks at the edges of the plan that picks their kernel (fl_dec16, fl_attn, fl_pf) and splits: splits of one tile, a last split of a few
 keys, 8, 9, 16 and more splits (each merge build), blocks and windows whose first or last rows see no key of a split.
 Oracle and bars as test_gpu_flint.py: attn_pf within 1e-5."""
 import pytest
@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 # (sliding, pos0, T)
 CASES = [(False, 27, 5), (False, 28, 5), (False, 250, 16), (False, 600, 5), (False, 1500, 17), (False, 2040, 8),
          (False, 33, 32), (False, 224, 33), (False, 2000, 64), (False, 2011, 100), (False, 600, 256),
-         (True, 600, 5), (True, 1030, 31), (True, 511, 97), (True, 1000, 256)]
+         (False, 2046, 1), (False, 2047, 2), (False, 3071, 1), (False, 3072, 2), (False, 3400, 20), (False, 33, 128),
+         (True, 520, 1), (True, 1024, 2), (True, 600, 5), (True, 1030, 31), (True, 511, 97), (True, 1000, 256)]
 
 
 @pytest.mark.parametrize("fmt", [F32, F16])
