@@ -337,13 +337,18 @@ __global__ void __launch_bounds__(NTH, NWV == 4 ? 2 : 1) attn_f32(const float* _
 }  // namespace
 
 Attn32Plan attn32_plan(int T, int n, int start) {
-    // the window's tiles dealt round robin, four per work-group, to at most 248 work-groups per kv head (registers
-    // held to 256 per lane, so two work-groups share a CU past 256 of them): at 16,384 positions (128 per kv head) the
-    // core takes 21.3-21.5 us, with two tiles per work-group (248) 24.7 us; per cfg5 verify three or five tiles per
-    // work-group measured 30.0 and 27.0 us against 24.5, at most 108 work-groups 24.9 us. Every work-group holds keys
-    // of every row, so the merge reads all (span 0)
+    // the window's tiles dealt round robin. From 12,289 positions on four per work-group, to at most 248 work-groups per
+    // kv head (registers held to 256 per lane, so two work-groups share a CU past 256 of them): at 16,384 positions (128
+    // per kv head) the core takes 21.3-21.5 us, with two tiles per work-group (248) 24.7 us; per cfg5 verify three or
+    // five tiles per work-group measured 30.0 and 27.0 us against 24.5, at most 108 work-groups 24.9 us. Shorter
+    // windows one (up to 64 tiles: the partials of the smallest store, 4,096 positions, hold 66 splits), two or three,
+    // which still leaves at most one work-group per CU: a decode of one / four tokens on four and on these at 200 / 700 /
+    // 4,096 / 12,000 positions 19.0 / 15.6 / 14.3 / 17.5 and 19.7 / 16.3 / 16.9 / 19.6 -> 7.9 / 8.2 / 10.9 / 15.1 and
+    // 8.6 / 8.9 / 13.0 / 18.8 us. Every work-group holds keys of every row, so the merge reads all (span 0)
     const int kend = n + T - 1;
-    int nch = (kend - start / TILE * TILE) / 128;
+    const int keys = kend - start / TILE * TILE, tiles = (keys + TILE - 1) / TILE;
+    const int per = tiles <= 64 ? 1 : tiles <= 256 ? 2 : (tiles + 127) / 128;
+    int nch = per < 4 ? (tiles + per - 1) / per : keys / 128;
     nch = nch > 248 ? 248 : nch < 1 ? 1 : nch;
     return Attn32Plan{0, nch, 0, (T + 3) / 4};
 }
