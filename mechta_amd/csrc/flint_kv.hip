@@ -36,6 +36,26 @@ namespace {
 #define FL_DEC_NCH 48     // decode: splits per kv head at most (32,768 positions: 48 against 32 / 64 / 96 splits
                           // 17.9-18.3 against 19.2 / 18.3-18.5 / 19.7 us per f16 call)
 #endif
+#ifndef FL_FUSE_NCH
+#define FL_FUSE_NCH 8     // decode with the merge fused (short spans): splits per kv head at most
+#endif
+#ifndef FL_FUSE_SPLIT
+#define FL_FUSE_SPLIT 80  // decode with the merge fused: positions per split at least (at 544 positions: 6 splits;
+                          // against 8 / 7 / 5 / 4 splits 9.8 against 10.7 / 9.8 / 10.0 / 10.7 us per f32 call, 8.6
+                          // against 8.8 / 8.6 / 8.5 / 8.8 us per f16 call)
+#endif
+// Decodes of spans up to these many positions merge in the kernel; longer ones launch the merge. One token on a full
+// layer, us per call with the merge in the kernel against two launches: f32 at 320 / 384 / 448 / 512 / 768 / 2,048
+// positions 9.1 / 9.5 / 10.1 / 10.2 / 10.4 / 13.0 against 9.0 / 9.5 / 9.8 / 9.9 / 9.6 / 10.7; f16 8.1 / 8.3 / 8.6 / 8.8
+// / 9.0 / 10.4 against 8.2 / 8.6 / 8.8 / 9.0 / 8.7 / 9.2; at 256 positions 9.0 / 8.2 against 10.7 / 10.2 (f32 / f16).
+// A sliding layer's 513-544 positions: 9.8 / 8.6 against 8.9 / 8.3.
+#ifndef FL_FUSE_SPAN_F32
+#define FL_FUSE_SPAN_F32 384
+#endif
+#ifndef FL_FUSE_SPAN_F16
+#define FL_FUSE_SPAN_F16 512
+#endif
+
 // Decodes (1-2 tokens) of more than these many positions take fl_dec16, whose waves keep more of the keys in flight;
 // shorter ones fl_attn, whose splits of one tile finish sooner. One token on a full layer, us per call, on fl_dec16 (up
 // to 384 positions f32 and 512 f16 with the merge in the kernel) / fl_attn: f32 at 100 / 544 / 1,200 / 2,040 / 3,060
@@ -722,7 +742,8 @@ template <int FMT, int NBUF>
 __global__ void __launch_bounds__(256) fl_dec16(const void* __restrict__ kplane, const void* __restrict__ vplane,
                                                 size_t plane_elems, int rows, const float* __restrict__ q, int T,
                                                 int pos0, int win, float scale2, int klo, int span, int nch,
-                                                float* __restrict__ part) {
+                                                float* __restrict__ part, unsigned* __restrict__ arrivals,
+                                                const float* __restrict__ sinks, float* __restrict__ out) {
     constexpr int BPE = FMT == 1 ? 4 : 2;
     const int c = blockIdx.x % nch, kvh = blockIdx.x / nch;
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, r16 = lane & 15;
@@ -885,6 +906,13 @@ __global__ void __launch_bounds__(256) fl_dec16(const void* __restrict__ kplane,
         ml[w][1][r16] = l_run;
     }
     __syncthreads();
+    // With the merge fused (arrivals != NULL, few splits), the partial is stored device-coherent (scope bit sc1,
+    // through the XCD's L2) and the kv head's last work-group to arrive merges them all; no work-group waits.
+    const bool fused = arrivals != nullptr;
+    auto put = [&](float* p, float x) {
+        if (fused) __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else *p = x;
+    };
     const size_t rbase = (size_t)kvh * T * GQA;
     {
         // every wave combines dims 16cc .. 16cc + 15 of cc = 2w, 2w + 1 for its lane's rows 4g + r: the rows' factors
@@ -914,7 +942,7 @@ __global__ void __launch_bounds__(256) fl_dec16(const void* __restrict__ kplane,
                     float o = 0.f;
 #pragma unroll
                     for (int ww = 0; ww < 4; ww++) o += f[ww][r] * x[c2][ww][r];
-                    p[16 * (2 * w + c2)] = o;
+                    put(p + 16 * (2 * w + c2), o);
                 }
             }
         }
@@ -927,9 +955,61 @@ __global__ void __launch_bounds__(256) fl_dec16(const void* __restrict__ kplane,
         for (int ww = 0; ww < 4; ww++)
             Lt += ml[ww][0][r16] == NEG_INF ? 0.f : exp2f(ml[ww][0][r16] - M) * ml[ww][1][r16];
         float* p = part + ((rbase + r16) * nch + c) * PART;
-        p[0] = M;
-        p[1] = Lt;
+        put(p, M);
+        put(p + 1, Lt);
     }
+    if (!fused) return;
+    // every wave's partial stores complete before the work-group barrier; wave 0 then releases at agent scope: the
+    // partial happens before the arrival that counts it, and the kv head's last arrival acquires, so its merge reads
+    // every partial
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    __shared__ int last;
+    if (w == 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        int l = 0;
+        if (lane == 0) {
+            l = __hip_atomic_fetch_add(arrivals + kvh, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                (unsigned)(nch - 1);
+            if (l) __hip_atomic_store(arrivals + kvh, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            last = l;
+        }
+        if (__builtin_amdgcn_readfirstlane(l)) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
+    __syncthreads();  // the other waves see the acquiring wave's view through the work-group barrier
+    if (!last) return;
+    // the kv head's last work-group: the merge of fl_merge for its rows (row = token * 8 + head of the kv head, T * 8
+    // <= 16), thread = (row, 8 dims), every split's partial loaded in one round trip (device-coherent loads)
+    const int row = tid >> 4, d0 = (tid & 15) * 8;
+    if (row >= T * GQA) return;
+    const int head = kvh * GQA + (row & 7), t = row >> 3;
+    const rsrc_t pr = plane_rsrc(part + (size_t)kvh * T * GQA * nch * PART, (unsigned)(T * GQA * nch * PART * 4));
+    f32x4 hd[FL_FUSE_NCH], a0[FL_FUSE_NCH], a1[FL_FUSE_NCH];
+#pragma unroll
+    for (int cj = 0; cj < FL_FUSE_NCH; cj++) {
+        const unsigned off = cj < nch ? (unsigned)(((row * nch + cj) * PART) * 4) : 0x7FFFFFF0u;
+        const unsigned oa = off + (PACC + d0) * 4;
+        hd[cj] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(pr, off, 0, LOAD_SC1));
+        a0[cj] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(pr, oa, 0, LOAD_SC1));
+        a1[cj] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(pr, oa + 16, 0, LOAD_SC1));
+    }
+    const float sk = sinks ? sinks[head] * LOG2E : NEG_INF;
+    float M = sk;
+#pragma unroll
+    for (int cj = 0; cj < FL_FUSE_NCH; cj++)
+        if (cj < nch) M = fmaxf(M, hd[cj].x);
+    f32x4 s0 = f32x4{}, s1 = f32x4{};
+    float L = sinks && M != NEG_INF ? exp2f(sk - M) : 0.f;
+#pragma unroll
+    for (int cj = 0; cj < FL_FUSE_NCH; cj++) {
+        const float e = cj < nch && hd[cj].x != NEG_INF ? exp2f(hd[cj].x - M) : 0.f;
+        L += e * hd[cj].y;
+        s0 += e * a0[cj];
+        s1 += e * a1[cj];
+    }
+    float* o = out + ((size_t)t * QH + head) * HD + d0;
+    *(f32x4*)o = s0 / L;
+    *(f32x4*)(o + 4) = s1 / L;
 }
 
 // Merge for few splits (prefill blocks): 8 rows (token, head) per work-group of 256 threads, 4 dims per thread, the
@@ -980,7 +1060,15 @@ Plan plan(int fmt, int pos0, int T, int win) {
     int span = pos0 + T - klo;
     int nrb = (T + 3) / 4;
     int nch, blk = 4;
-    if (T <= 2 && span > (fmt == 1 ? FL_DEC_SPAN_F32 : FL_DEC_SPAN_F16)) {  // fl_dec16
+    int fused = 0;
+    if (T <= 2 && span <= (fmt == 1 ? FL_FUSE_SPAN_F32 : FL_FUSE_SPAN_F16)) {  // fl_dec16 merging its own partials: one
+        // launch less; fl_attn and a merge take 7.5 against 9.1 us back to back at 250 positions, but a whole step (32.6
+        // us, a sliding and a full layer) 36.1
+        blk = T;
+        nch = span / FL_FUSE_SPLIT;
+        nch = nch > FL_FUSE_NCH ? FL_FUSE_NCH : nch;
+        fused = 1;
+    } else if (T <= 2 && span > (fmt == 1 ? FL_DEC_SPAN_F32 : FL_DEC_SPAN_F16)) {  // fl_dec16
         blk = T;
         nch = span / FL_DEC_SPLIT;
         nch = nch > FL_DEC_NCH ? FL_DEC_NCH : nch;
@@ -1026,10 +1114,10 @@ Plan plan(int fmt, int pos0, int T, int win) {
         if (blk == 4) span = (span + TILE - 1) / TILE * TILE;  // whole tiles divide evenly
     }
     nch = nch < 1 ? 1 : nch;
-    return Plan{klo, span, nch, nrb, blk};
+    return Plan{klo, span, nch, nrb, blk, fused};
 }
 
-size_t ws_floats() { return (size_t)KVH * WS_ROWS * PART; }
+size_t ws_floats() { return (size_t)KVH * WS_ROWS * PART + WS_ARRIVALS; }
 
 hipError_t launch_attn(int fmt, const void* kp, const void* vp, int rows, const float* q, int T, int pos0, int win,
                        const Plan& p, float* ws, const float* sinks, float* out, hipStream_t st) {
@@ -1039,11 +1127,15 @@ hipError_t launch_attn(int fmt, const void* kp, const void* vp, int rows, const 
     const dim3 grid(p.nrb * p.nch * KVH);
     const Launch L{st};
     hipError_t e;
+    // arrival counters of the fused decode merge, zero between launches, after the partials
+    unsigned* arr = p.fused ? (unsigned*)(ws + (size_t)KVH * WS_ROWS * PART) : nullptr;
+    if (p.fused && p.nch > FL_FUSE_NCH) return hipErrorInvalidValue;
     if (p.blk <= 2) {  // decode (and 2-token steps): 16-row kernel
         e = fmt == 1 ? launch(fl_dec16<1, FL_DEC_BUF>, dim3(p.nch * KVH), dim3(256), L, kp, vp, pe, rows, q, T, pos0,
-                              win, scale2, p.klo, p.span, p.nch, ws)
+                              win, scale2, p.klo, p.span, p.nch, ws, arr, sinks, out)
                      : launch(fl_dec16<0, FL_DEC_BUF>, dim3(p.nch * KVH), dim3(256), L, kp, vp, pe, rows, q, T, pos0,
-                              win, scale2, p.klo, p.span, p.nch, ws);
+                              win, scale2, p.klo, p.span, p.nch, ws, arr, sinks, out);
+        if (p.fused) return e;
     } else if (p.blk == 4) {  // blocks of 4 tokens
         e = fmt == 1 ? launch(fl_attn<1, 2>, grid, dim3(256), L, kp, vp, pe, rows, q, T, pos0, win, scale2, p.klo,
                               p.span, p.nch, p.nrb, ws)
