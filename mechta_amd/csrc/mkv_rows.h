@@ -57,11 +57,13 @@ __global__ void __launch_bounds__(256) rows_tile(E* __restrict__ plane, size_t p
         constexpr int NG = PB / EPC;
         auto group = [&](int g, int e) { return plane + (size_t)(e / HD) * plane_elems + (size_t)(q0 / EPC + g) * (EPC * HD) + (size_t)(e % HD) * EPC; };
         if constexpr (DIR == 1) {
+            // rows outside the range are loaded as its nearest one and not stored: a load behind a branch each took the f32
+            // build to 230 registers and one load at a time (100 positions 4.5 us, 1,000 4.8; now 2.3 and 2.6)
             u32x4 x[IT];
 #pragma unroll
             for (int k = 0; k < IT; k++) {
-                const int c = tid + 256 * k, p = q0 + c / CPR, e = (c % CPR) * EPC;
-                if (p >= p0 && p < p1) x[k] = *(const u32x4*)(rows + (size_t)(p - p0) * ROWE + e);
+                const int c = tid + 256 * k, p = min(max(q0 + c / CPR, p0), p1 - 1), e = (c % CPR) * EPC;
+                x[k] = *(const u32x4*)(rows + (size_t)(p - p0) * ROWE + e);
             }
 #pragma unroll
             for (int k = 0; k < IT; k++) {
