@@ -634,28 +634,44 @@ hipError_t launch_small_prefill(const Geom& g, const void* base, int layer, cons
                   32 * p.nzb, p.nzb);
 }
 
+int merge_width(int ntok, int n, int start, int span, int nch) {
+    // few chunks, or many rows (prefill blocks) over up to two groups of chunks: a row per 64 threads (a 128-token
+    // block at 28,000 positions, 32 splits, 87.8 against 94.2 us per step; with 64 splits, four groups, slower than
+    // decode_combine: 68.4 against 63.0 us); with few rows decode_combine's smaller work-groups are faster (32 tokens of
+    // the f32 store at 4,000 positions, 32 splits: 30.8 against 34.3 us). Chunks: the ones that hold a key of the last
+    // token's window, not the call's splits (63 tokens of the f32 store at 9,000 positions, start 8,500, 32 splits, 2 of
+    // them in the window: decode_combine's 4,032 work-groups 50.3 us per call, merge_few<4> 41.2)
+    int c0, c1;
+    chunk_range(start, n + ntok - 1, span, nch, c0, c1);
+    const int m = c1 - c0;
+    if (m <= 4) return 4;
+    if (m <= 8) return 8;  // the 8 splits of a 512-token block: 12.2 against 14.5 us with the 16-chunk build
+    if (m <= MERGE_FEW) return MERGE_FEW;
+    if (ntok >= 64 && m <= 2 * MERGE_FEW) return 2 * MERGE_FEW;
+    return m <= 16 * 9 ? 16 * 9 : 16 * MERGE_JMAX;
+}
+
 template <bool H16>
 hipError_t merge_as(const float* part, int rpk, int ntok, int n, int start, int span, int nch, const float* gate,
                     void* out, const Launch& L) {
     if (nch > 16 * MERGE_JMAX) return hipErrorInvalidValue;
-    // few chunks, or many rows (prefill blocks) over up to two groups of chunks: a row per 64 threads (a 128-token
-    // block at 28,000 positions, 32 splits, 87.8 against 94.2 us per step; with 64 splits, four groups, slower than
-    // decode_combine: 68.4 against 63.0 us); with few rows decode_combine's smaller work-groups are faster (32 tokens of
-    // the f32 store at 4,000 positions, 32 splits: 30.8 against 34.3 us)
     const dim3 few((ntok * QH + 3) / 4), rows(ntok * QH, HD / 64);
-    if (nch <= 4)
-        return launch(merge_few<false, H16, 4>, few, dim3(256), L, part, rpk, ntok, n, start, span, nch, gate, out);
-    if (nch <= 8)  // the 8 splits of a 512-token block: 12.2 against 14.5 us with the 16-chunk build
-        return launch(merge_few<false, H16, 8>, few, dim3(256), L, part, rpk, ntok, n, start, span, nch, gate, out);
-    if (nch <= MERGE_FEW)
-        return launch(merge_few<false, H16, MERGE_FEW>, few, dim3(256), L, part, rpk, ntok, n, start, span, nch, gate,
-                      out);
-    if (ntok >= 64 && nch <= 2 * MERGE_FEW)
-        return launch(merge_few<true, H16, MERGE_FEW>, few, dim3(256), L, part, rpk, ntok, n, start, span, nch, gate,
-                      out);
-    if (nch <= 16 * 9)
-        return launch(decode_combine<9, H16>, rows, dim3(256), L, part, rpk, n, start, span, nch, gate, out);
-    return launch(decode_combine<MERGE_JMAX, H16>, rows, dim3(256), L, part, rpk, n, start, span, nch, gate, out);
+    switch (merge_width(ntok, n, start, span, nch)) {
+        case 4:
+            return launch(merge_few<false, H16, 4>, few, dim3(256), L, part, rpk, ntok, n, start, span, nch, gate, out);
+        case 8:
+            return launch(merge_few<false, H16, 8>, few, dim3(256), L, part, rpk, ntok, n, start, span, nch, gate, out);
+        case MERGE_FEW:
+            return launch(merge_few<false, H16, MERGE_FEW>, few, dim3(256), L, part, rpk, ntok, n, start, span, nch, gate,
+                          out);
+        case 2 * MERGE_FEW:
+            return launch(merge_few<true, H16, MERGE_FEW>, few, dim3(256), L, part, rpk, ntok, n, start, span, nch, gate,
+                          out);
+        case 16 * 9:
+            return launch(decode_combine<9, H16>, rows, dim3(256), L, part, rpk, n, start, span, nch, gate, out);
+        default:
+            return launch(decode_combine<MERGE_JMAX, H16>, rows, dim3(256), L, part, rpk, n, start, span, nch, gate, out);
+    }
 }
 
 hipError_t launch_merge(const float* part, int rpk, int ntok, int n, int start, int span, int nch, const float* gate,

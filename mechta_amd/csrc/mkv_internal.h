@@ -164,6 +164,9 @@ bool small_prefill_pays(int T, int n, int start);  // T > SMALL_PREFILL_MAX: fas
 size_t small_prefill_ws_floats(int T, int nch);
 hipError_t launch_small_prefill(const Geom& g, const void* base, int layer, const float* q, int T, int n, int start,
                                 float scale, const SmallPlan& p, float* ws, const Launch& L);
+// The merge build of a call, by the most chunks it takes: 4, 8 or 16 (merge_few), 32 (merge_few, two groups), 144 or 256
+// (decode_combine).
+int merge_width(int ntok, int n, int start, int span, int nch);
 // Merge of split-K partials laid out [kvh][row < rpk][chunk < nch][PART], row = token*8 + head of the kv head:
 // out[t][head] for t < ntok over the chunks (chunk_lo of span, nch) holding a key of [start, n + t), optional gate;
 // out is f32, or with h16 f16 bits rounded to nearest even (attn_gate16).
