@@ -57,9 +57,11 @@ __global__ void __launch_bounds__(NTH, NWV == 4 ? 2 : 1) attn_f32(const float* _
                                                 float* __restrict__ part, const float* __restrict__ akn,
                                                 const float* __restrict__ av, const float* __restrict__ atab, int apos,
                                                 int antok) {
-    // XCD-aware order: the token blocks that stream the same keys on one XCD's L2
+    // XCD order only where each XCD gets as many work-groups: no two share keys here (one token block), and a grid that is
+    // no multiple of 8, in it, takes longer (1 token at 30,000 positions, 468 work-groups: 30.3 against 28.7 us; 2: 31.8
+    // against 30.8)
     const int G = gridDim.x, L = blockIdx.x;
-    const int W = xcd_order(L, G);
+    const int W = G % NXCD == 0 ? xcd_order(L, G) : L;
     const int ncg = nch - c0;
     const int rb = W % nrb, c = c0 + (W / nrb) % ncg, kvh = W / nrb / ncg;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, s = lane >> 5, r32 = lane & 31;
