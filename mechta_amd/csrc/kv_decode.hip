@@ -614,7 +614,7 @@ bool small_prefill_pays(int T, int n, int start) {
     if (T > 256) return false;  // no faster there (512 tokens at 300 positions 31 against 27-29 us)
     const SmallPlan p = small_prefill_plan(T, n, start);
     int other;
-    (void)prefill_plan(T, n, &other);
+    (void)prefill_plan(T, n, start, &other);
     return 1030 + 125 * ((p.d.nu + p.d.nch - 1) / p.d.nch) < other;
 }
 

@@ -544,17 +544,21 @@ __global__ void __launch_bounds__(P32_NW * 64) prefill_f32(const float* __restri
 // at 28,000 positions took 95 us on 64 work-groups, 64 us on 256. The workspace bound is tokens x splits <= 4,096.
 constexpr int PF_MAXCH = 64;
 // The cheapest split count of one work-group shape by a model of the call (0.01 us): what does not depend on the splits,
-// a wave's tiles, and what each split adds to the merge and in partials written and read back.
-static PrefillPlan best_splits(int T, int kend, int pt, int ks, int& cost) {
-    const int blocks = 2 * ((T + pt - 1) / pt), tiles = (kend + 31) / 32;
-    int most = 256 / blocks;  // at most about one work-group per CU
+// a wave's tiles, and what each split adds in partials written (20 of 55) and read back by the merge, which takes the
+// splits with keys from start on.
+static PrefillPlan best_splits(int T, int kend, int start, int ks, int& cost) {
+    const int pt = 32 / ks, blocks = (T + pt - 1) / pt, tiles = (kend + 31) / 32;
+    int most = 128 / blocks;  // at most about one work-group per CU
     most = most > PF_MAXCH ? PF_MAXCH : most < 1 ? 1 : most;
+    const int below = (int)(100LL * start / kend);  // of 100 tiles, the masked ones below the window
+    const int per = T * (55 - 35 * below / 100) + 2000;
     PrefillPlan p{kend, 1, ks};
     cost = INT_MAX;
     for (int nch = 1; nch <= most && (nch == 1 || nch * ks <= tiles); nch++) {
         const int s = (tiles + nch * ks - 1) / (nch * ks);  // tiles of a wave
-        const int t = ks == 1 ? 1100 + 135 * s : 1230 + 145 * s + (s > 40 ? 50 * (s - 40) : 0);
-        const int c = t + nch * T * 55 / 100 + 20 * nch;
+        // two groups: a masked tile costs more
+        const int t = ks == 1 ? 1100 + 135 * s : 1230 + 145 * s + s * below * 40 / 100 + (s > 40 ? 50 * (s - 40) : 0);
+        const int c = t + nch * per / 100;
         if (c < cost) {
             cost = c;
             p.nch = nch;
@@ -563,7 +567,7 @@ static PrefillPlan best_splits(int T, int kend, int pt, int ks, int& cost) {
     return p;
 }
 
-PrefillPlan prefill_plan(int T, int n, int* us100) {
+PrefillPlan prefill_plan(int T, int n, int start, int* us100) {
     // Measured per call with merge and gate. 512 tokens at 1,000 / 4,000 / 9,000 / 16,000 / 28,000 positions: one key group
     // 42.4 / 62.1 / 94.8 / 141 / 224, two 36.2 / 57.2 / 93.1 / 144 / 245 us: two groups read each tile for half as many rows
     // (which tells on long splits, where the card is power limited) and save half the partials. Splits, two groups: 64
@@ -571,22 +575,29 @@ PrefillPlan prefill_plan(int T, int n, int* us100) {
     // on 16 / 8 32.5 / 26.0 us.
     const int kend = n + T - 1;
     int c1, c2;
-    const PrefillPlan p1 = best_splits(T, kend, PfGeom<1>::PT, 1, c1), p2 = best_splits(T, kend, PfGeom<2>::PT, 2, c2);
+    const PrefillPlan p1 = best_splits(T, kend, start, 1, c1), p2 = best_splits(T, kend, start, 2, c2);
     if (us100) *us100 = c2 <= c1 ? c2 : c1;
     return c2 <= c1 ? p2 : p1;
 }
 
-PrefillPlan prefill32_plan(int T, int n) {
+PrefillPlan prefill32_plan(int T, int n, int start) {
     // As best_splits (0.01 us): 2.55 us per tile of a work-group against the partials and the merge, whose kernel for more
-    // than 16 splits takes about 3 us longer. 5 tokens at 1,000 / 9,000 / 20,000 positions 17.9 / 27.6 / 44.5 us on at most
-    // 64 splits of at least 64 positions, 14.4 / 21.7 / 32.7 on these; 64 tokens at 1,000 positions on 8 / 16 / 32 splits
-    // 26.1 / 24.6 / 31.4, at 4,000 59.5 / 41.6 / 38.4 us.
+    // than 16 splits in the window takes about 3 us longer. 5 tokens at 1,000 / 9,000 / 20,000 positions 17.9 / 27.6 / 44.5
+    // us on at most 64 splits of at least 64 positions, 14.4 / 21.7 / 32.7 on these; 64 tokens at 1,000 positions on 8 / 16 /
+    // 32 splits 26.1 / 24.6 / 31.4, at 4,000 59.5 / 41.6 / 38.4 us; at 2,000 with a window of 500 on 16 / 20 / 32 27.0 / 24.6 /
+    // 22.6.
     const int kend = n + T - 1, tiles = (kend + 31) / 32;
     int most = 256 / (KVH * ((T + P32_PT - 1) / P32_PT));  // at most about one work-group per CU
     most = most < 1 ? 1 : most;
     int best = INT_MAX, nch = 1;
+    // The merge reads the splits with keys of the window, and the stores of the others cost nothing measurable; with a window
+    // the mean of a split's longest and average tiles fits best (121 windows of 5-256 tokens at 64-9,000 positions, each on
+    // 10 split counts: 1.5% on average behind the best of them; splits as without a window 2-3%, up to 17%)
+    const long long seen = kend - start;
+    const int per = (int)((T < 64 ? T * 45 : T * 55 + 800) * seen / kend);
     for (int k = 1; k <= most && k <= tiles; k++) {
-        const int c = 255 * tiles / k + (T < 64 ? k * T * 45 / 100 : k * T * 55 / 100 + 8 * k) + (k > 16 ? 300 : 0);
+        const int len = start > 0 ? 255 * tiles / k / 2 + 255 * ((tiles + k - 1) / k) / 2 : 255 * tiles / k;
+        const int c = len + k * per / 100 + (k * seen > 16LL * kend ? 300 : 0);
         if (c < best) {
             best = c;
             nch = k;

@@ -438,7 +438,7 @@ int mkv_prefill(mkv_t* h, int layer, const float* q, int T, int n, int start, fl
     } else {
         // f16: attn_fa_mx's arithmetic on 32-token work-groups; f32: 16-token work-groups, f32-class arithmetic
         const bool f16 = h->g.fmt == MKV_F16;
-        const PrefillPlan p = f16 ? prefill_plan(T, n) : prefill32_plan(T, n);
+        const PrefillPlan p = f16 ? prefill_plan(T, n, start) : prefill32_plan(T, n, start);
         if (prefill_ws_floats(T, p.nch) > h->pws_floats) return fail(MKV_E_ARG, "mkv_prefill: workspace");
         span = p.span;
         nch = p.nch;

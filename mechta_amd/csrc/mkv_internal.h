@@ -190,12 +190,12 @@ struct PrefillPlan {
     int span, nch;  // splits of [0, span) as chunk_lo
     int ks;         // f16: key groups per work-group (1 or 2)
 };
-PrefillPlan prefill_plan(int T, int n, int* us100 = nullptr);  // us100: the plan's modelled time (0.01 us)
+PrefillPlan prefill_plan(int T, int n, int start, int* us100 = nullptr);  // us100: the plan's modelled time (0.01 us)
 size_t prefill_ws_floats(int T, int nch);
 hipError_t launch_prefill(const Geom& g, const void* base, int layer, const float* q, int T, int n, int start,
                           float scale, const PrefillPlan& p, float* ws, const Launch& L);
 // f32 store: prefill_f32 (16-token work-groups over an LDS ring, f32-class arithmetic)
-PrefillPlan prefill32_plan(int T, int n);
+PrefillPlan prefill32_plan(int T, int n, int start);
 hipError_t launch_prefill_f32(const Geom& g, const void* base, int layer, const float* q, int T, int n, int start,
                               float scale, const PrefillPlan& p, float* ws, const Launch& L);
 

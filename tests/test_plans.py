@@ -27,3 +27,31 @@ def merge_width(ntok, n, start, span, nch):
 def test_merge_takes_the_window_chunks(ntok, n, start, nch, want):
     """By the chunks that hold a key of the window, not by the call's splits."""
     assert merge_width(ntok, n, start, n + ntok - 1, nch) == want
+
+
+class PrefillPlan(ctypes.Structure):
+    _fields_ = [("span", I), ("nch", I), ("ks", I)]
+
+
+def prefill_plan(T, n, start=0):
+    """prefill_f16's splits and key groups per work-group (1 or 2)."""
+    return fn("_ZN3mkv12prefill_planEiiiPi", PrefillPlan)(T, n, start, None)
+
+
+def prefill32_plan(T, n, start=0):
+    return fn("_ZN3mkv14prefill32_planEiii", PrefillPlan)(T, n, start)
+
+
+@pytest.mark.parametrize("T,n,start,least", [(63, 2000, 1500, 24), (64, 2000, 1500, 22), (48, 4000, 3500, 32),
+                                             (80, 4000, 3500, 22), (16, 2000, 1500, 32)])
+def test_f32_window_takes_more_splits(T, n, start, least):
+    """A merge that reads two or three chunks does not pay for the others: on the splits of the same call without a window
+    (mostly 16), these took 4-20% longer than on `least` splits or more."""
+    assert prefill32_plan(T, n, start).nch >= least
+
+
+@pytest.mark.parametrize("T,n,start", [(320, 9000, 8500), (384, 9000, 8500), (512, 6000, 5500), (184, 20000, 19500),
+                                       (96, 45000, 44500)])
+def test_f16_window_takes_one_group(T, n, start):
+    """Two groups save half of a merge that reads little: 4-10% slower there with a window."""
+    assert prefill_plan(T, n, start).ks == 1
