@@ -545,7 +545,7 @@ __global__ void __launch_bounds__(P32_NW * 64) prefill_f32(const float* __restri
 constexpr int PF_MAXCH = 64;
 // The cheapest split count of one work-group shape by a model of the call (0.01 us): what does not depend on the splits,
 // a wave's tiles, and what each split adds in partials written (20 of 55) and read back by the merge, which takes the
-// splits with keys from start on.
+// splits with keys from start on; from 32 splits on a split costs half.
 static PrefillPlan best_splits(int T, int kend, int start, int ks, int& cost) {
     const int pt = 32 / ks, blocks = (T + pt - 1) / pt, tiles = (kend + 31) / 32;
     int most = 128 / blocks;  // at most about one work-group per CU
@@ -556,23 +556,32 @@ static PrefillPlan best_splits(int T, int kend, int start, int ks, int& cost) {
     cost = INT_MAX;
     for (int nch = 1; nch <= most && (nch == 1 || nch * ks <= tiles); nch++) {
         const int s = (tiles + nch * ks - 1) / (nch * ks);  // tiles of a wave
-        // two groups: a masked tile costs more
-        const int t = ks == 1 ? 1100 + 135 * s : 1230 + 145 * s + s * below * 40 / 100 + (s > 40 ? 50 * (s - 40) : 0);
-        const int c = t + nch * per / 100;
+        const int c = (ks == 1 ? 1100 + 135 * s : 1230 + 145 * s) + (nch <= 32 ? nch : 16 + nch / 2) * per / 100;
         if (c < cost) {
             cost = c;
             p.nch = nch;
         }
     }
+    // The card is power limited on long calls. One group: a block of 32 tokens computes up to 16 absent ones more than
+    // blocks of 16. Two groups: each tile read for half as many rows, and a masked tile costs more.
+    const int s = (tiles + p.nch * ks - 1) / (p.nch * ks);
+    if (ks == 1) cost += (blocks * 32 - (T + 15) / 16 * 16) * tiles * 40 / 1000;
+    else cost += s * below * 40 / 100 + (T > 256 ? s * (T - 256) * 24 / 512 : 0) + (s > 32 ? 60 * (s - 32) : 0);
     return p;
 }
 
 PrefillPlan prefill_plan(int T, int n, int start, int* us100) {
-    // Measured per call with merge and gate. 512 tokens at 1,000 / 4,000 / 9,000 / 16,000 / 28,000 positions: one key group
-    // 42.4 / 62.1 / 94.8 / 141 / 224, two 36.2 / 57.2 / 93.1 / 144 / 245 us: two groups read each tile for half as many rows
-    // (which tells on long splits, where the card is power limited) and save half the partials. Splits, two groups: 64
-    // tokens at 4,000 positions on 32 / 16 / 8 splits 32.7 / 26.4 / 26.2, at 9,000 34.4 / 31.5 / 38.7, 128 tokens at 2,000
-    // on 16 / 8 32.5 / 26.0 us.
+    // Two key groups save half the partials and read each tile for half as many rows, which tells on long splits, where the
+    // card is power limited, and sooner where the keys come from HBM. Time of two groups over one, per call with the merge,
+    // keys from HBM (as many layers in turn as 640 MB hold) / from the last-level cache:
+    //   512 tokens at 1,000, 4,000, 7,500, 9,000, 12,000, 28,000 positions .92 .95 1.02 1.08 1.08 1.10 / .91 .93 .97 .98 1.00 1.05
+    //   256 tokens at 1,000, 9,000, 16,000, 20,000, 24,000, 28,000         .91 .95 .98 1.02 1.05 1.07 / .91 .91 .96 .97 .99 1.00
+    //   200 tokens at 2,000, 9,000, 20,000, 28,000, 36,000                 .91 .82 .93 .96 1.00       / .90 .81 .90 .94
+    //   128 tokens at 2,000, 9,000, 28,000, 45,000, 60,000                 .89 .90 .94 1.00 1.05      / .88 .88 .92
+    //    64 tokens at 3,000, 28,000, 60,000, 90,000, 120,000               .88 .99 1.01 1.07 1.11     / .87 .97
+    // The line lies between the two crossings. Over 570 such pairs (64-512 tokens) the plan loses 0.1% on average against
+    // the faster group count, 4.4% at most from HBM and 6% from the cache. Splits, two groups: 64 tokens at 4,000 positions
+    // on 32 / 16 / 8 splits 32.7 / 26.4 / 26.2 us, at 9,000 34.4 / 31.5 / 38.7, 128 tokens at 2,000 on 16 / 8 32.5 / 26.0.
     const int kend = n + T - 1;
     int c1, c2;
     const PrefillPlan p1 = best_splits(T, kend, start, 1, c1), p2 = best_splits(T, kend, start, 2, c2);

@@ -55,3 +55,14 @@ def test_f32_window_takes_more_splits(T, n, start, least):
 def test_f16_window_takes_one_group(T, n, start):
     """Two groups save half of a merge that reads little: 4-10% slower there with a window."""
     assert prefill_plan(T, n, start).ks == 1
+
+
+# (tokens, positions, faster group count): pairs measured with the keys from HBM, 4% apart or more
+GROUPS = [(512, 9000, 1), (512, 12000, 1), (512, 28000, 1), (384, 14000, 1), (320, 16000, 1), (256, 24000, 1), (160, 45000, 1),
+          (128, 60000, 1), (96, 90000, 1), (64, 90000, 1), (64, 120000, 1), (512, 3000, 2), (384, 6000, 2), (256, 12000, 2),
+          (200, 9000, 2), (200, 28000, 2), (128, 28000, 2), (72, 28000, 2), (64, 16000, 2)]
+
+
+@pytest.mark.parametrize("T,n,ks", GROUPS)
+def test_key_groups(T, n, ks):
+    assert prefill_plan(T, n).ks == ks
