@@ -66,3 +66,20 @@ GROUPS = [(512, 9000, 1), (512, 12000, 1), (512, 28000, 1), (384, 14000, 1), (32
 @pytest.mark.parametrize("T,n,ks", GROUPS)
 def test_key_groups(T, n, ks):
     assert prefill_plan(T, n).ks == ks
+
+
+class FlintPlan(ctypes.Structure):
+    _fields_ = [(x, I) for x in ("klo", "span", "nch", "nrb", "blk", "fused")]
+
+
+def flint_plan(fmt, pos0, T, win=0):
+    """blk: 1-2 (fl_dec16), 4 (fl_attn), 32 (fl_pf)."""
+    return fn("_ZN3mkv5flint4planEiiii", FlintPlan)(fmt, pos0, T, win)
+
+
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("T,nch", [(5, 64), (12, 64), (24, 64), (48, 32)])
+def test_flint_long_spans_take_every_split(fmt, T, nch):
+    """Splits of a dozen tiles or more finish sooner the more there are, also where the longest is as long."""
+    p = flint_plan(fmt, 30000, T)
+    assert (p.blk, p.nch) == (32, nch)
