@@ -77,8 +77,7 @@ def flint_plan(fmt, pos0, T, win=0):
     return fn("_ZN3mkv5flint4planEiiii", FlintPlan)(fmt, pos0, T, win)
 
 
-@pytest.mark.parametrize("fmt", [0, 1])
-@pytest.mark.parametrize("T,nch", [(5, 64), (12, 64), (24, 64), (48, 32)])
+@pytest.mark.parametrize("fmt,T,nch", [(0, 5, 64), (0, 12, 64), (0, 24, 64), (0, 48, 32), (1, 12, 64), (1, 24, 64), (1, 48, 32)])
 def test_flint_long_spans_take_every_split(fmt, T, nch):
     """Splits of a dozen tiles or more finish sooner the more there are, also where the longest is as long."""
     p = flint_plan(fmt, 30000, T)
