@@ -611,7 +611,7 @@ bool small_prefill_pays(int T, int n, int start) {
     // prefill_f16: 64 tokens at 300 / 1,000 / 4,000 / 9,000 positions 11.6 / 13.9 / 21.1 / 32.8 against 17.4 / 19.0 / 26.2 /
     // 31.5 us, 128 tokens at 300 / 1,000 / 4,000 13.4 / 17.6 / 32.1 against 18.0 / 21.7 / 31.0, 256 tokens at 300 / 1,000
     // 18.5 / 24.4 against 21.8 / 26.2 us
-    if (T > 256) return false;  // no faster there (512 tokens at 300 positions 31 against 27-29 us)
+    if (T > SMALL_PAYS_MAX) return false;  // no faster there (512 tokens at 300 positions 31 against 27-29 us)
     const SmallPlan p = small_prefill_plan(T, n, start);
     int other;
     (void)prefill_plan(T, n, start, &other);
@@ -622,7 +622,7 @@ size_t small_prefill_ws_floats(int T, int nch) { return (size_t)KVH * 32 * ((T +
 
 hipError_t launch_small_prefill(const Geom& g, const void* base, int layer, const float* q, int T, int n, int start,
                                 float scale, const SmallPlan& p, float* ws, const Launch& L) {
-    if (g.fmt != 0 || T < 1) return hipErrorNotSupported;
+    if (g.fmt != 0 || T < 1 || T > SMALL_PAYS_MAX) return hipErrorNotSupported;
     char* b = (char*)base;
     void* kp = b + g.plane(layer, 0, 0) * g.plane_bytes();
     void* vp = b + g.plane(layer, 1, 0) * g.plane_bytes();

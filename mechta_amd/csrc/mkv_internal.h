@@ -155,6 +155,7 @@ hipError_t launch_decode_merge(int ntok, int n, int start, const DecodePlan& p, 
 // of 4 tokens over the decode's stages; partials [kvh][row < 32 nzb][nch][PART], then launch_merge. Larger blocks take the
 // same kernel where the context is short (small_prefill_pays): it has little to set up.
 constexpr int SMALL_PREFILL_MAX = 63;
+constexpr int SMALL_PAYS_MAX = 256;  // tokens the small-block kernel takes at most
 struct SmallPlan {
     DecodePlan d;
     int nzb;  // blocks of 4 tokens

@@ -82,3 +82,24 @@ def test_flint_long_spans_take_every_split(fmt, T, nch):
     """Splits of a dozen tiles or more finish sooner the more there are, also where the longest is as long."""
     p = flint_plan(fmt, 30000, T)
     assert (p.blk, p.nch) == (32, nch)
+
+
+class Geom(ctypes.Structure):
+    _fields_ = [("layers", I), ("ctx", I), ("fmt", I), ("plane_elems", ctypes.c_size_t)]
+
+
+class SmallPlan(ctypes.Structure):
+    _fields_ = [(x, I) for x in ("span", "nch", "c0", "s0", "nu", "nzb")]
+
+
+class Launch(ctypes.Structure):
+    _fields_ = [(x, ctypes.c_void_p) for x in ("s", "a", "b")]
+
+
+@pytest.mark.parametrize("fmt,T", [(0, 0), (0, 257), (0, 512), (1, 16)])
+def test_small_block_launcher_refuses(fmt, T):
+    """hipErrorNotSupported (801) before any launch: the store's format, and blocks of more than 256 tokens."""
+    launch = fn("_ZN3mkv20launch_small_prefillERKNS_4GeomEPKviPKfiiifRKNS_9SmallPlanEPfRKNS_6LaunchE")
+    g, p, s = Geom(1, 4096, fmt, 4096 * 256), SmallPlan(0, 2, 0, 0, 2, 64), Launch(None, None, None)
+    rc = launch(ctypes.byref(g), None, 0, None, T, 1, 0, ctypes.c_float(1.0), ctypes.byref(p), None, ctypes.byref(s))
+    assert rc == 801
