@@ -1,7 +1,7 @@
 """f16 prefill blocks of 64 tokens or more on the three kernels' edges: the small-block kernel (short contexts, up to 256
-tokens), and prefill_f16 with one or two key groups: splits of one tile, an odd tile left over for one group, ragged last
-blocks and tiles, key counts on both sides of the rules that pick. Bars as test_gpu_kvpath.py: attn_fa_mx at the task
-tolerance, selected tokens."""
+tokens), and prefill_f16 with one or two key groups: waves of three tiles and more, an odd tile left over for one group,
+ragged last blocks and tiles, key counts on both sides of the rules that pick. Bars as test_gpu_kvpath.py: attn_fa_mx at the
+task tolerance, selected tokens (test_gpu_prefill_paths.py holds the small-block kernel to its own f32-class bar)."""
 import numpy as np
 import pytest
 
@@ -10,9 +10,9 @@ from tests.helpers import assert_attn_close, gate_inputs, prefill_reference, q_i
 
 pytestmark = pytest.mark.gpu
 
-# (n0, T, start): short contexts and up to 256 tokens: the small-block kernel; 257 and more: two groups, down to one tile
-# per split; block edges at 16 and 32 tokens; windows; long contexts, where wide blocks take one group (256 tokens cross
-# over near 25,000 positions, 512 near 12,000)
+# (n0, T, start): short contexts and up to 256 tokens: the small-block kernel; 257 and more: two groups, down to three tiles
+# per wave; block edges at 16 and 32 tokens; windows; long contexts, where wide blocks take one group (256 tokens cross
+# over near 22,000 positions, 512 near 9,000)
 CASES = [(1, 64, 0), (2, 65, 0), (31, 79, 0), (160, 96, 0), (161, 97, 40), (700, 127, 0), (1000, 241, 500), (64, 256, 0),
          (1, 257, 0), (31, 300, 0), (33, 512, 0), (700, 273, 600), (5000, 511, 0), (6000, 128, 0), (9000, 200, 0),
          (9011, 500, 4000), (20000, 256, 0), (30000, 512, 0), (30001, 255, 0), (32000, 67, 31000)]
