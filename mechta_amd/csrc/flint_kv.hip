@@ -29,11 +29,8 @@ namespace {
 #ifndef FL_DEC_BUF
 #define FL_DEC_BUF 2      // decode: subtiles in registers per wave
 #endif
-#ifndef FL_DEC_SPLIT
-#define FL_DEC_SPLIT 32   // decode: positions per split at least
-#endif
 #ifndef FL_DEC_NCH
-#define FL_DEC_NCH 48     // decode: splits per kv head at most (32,768 positions: 48 against 32 / 64 / 96 splits
+#define FL_DEC_NCH 48     // decode on fl_dec16: splits per kv head (32,768 positions: 48 against 32 / 64 / 96 splits
                           // 17.9-18.3 against 19.2 / 18.3-18.5 / 19.7 us per f16 call)
 #endif
 #ifndef FL_FUSE_NCH
@@ -44,11 +41,14 @@ namespace {
                           // against 8 / 7 / 5 / 4 splits 9.8 against 10.7 / 9.8 / 10.0 / 10.7 us per f32 call, 8.6
                           // against 8.8 / 8.6 / 8.5 / 8.8 us per f16 call)
 #endif
-// Decodes of spans up to these many positions merge in the kernel; longer ones launch the merge. One token on a full
-// layer, us per call with the merge in the kernel against two launches: f32 at 320 / 384 / 448 / 512 / 768 / 2,048
-// positions 9.1 / 9.5 / 10.1 / 10.2 / 10.4 / 13.0 against 9.0 / 9.5 / 9.8 / 9.9 / 9.6 / 10.7; f16 8.1 / 8.3 / 8.6 / 8.8
-// / 9.0 / 10.4 against 8.2 / 8.6 / 8.8 / 9.0 / 8.7 / 9.2; at 256 positions 9.0 / 8.2 against 10.7 / 10.2 (f32 / f16).
-// A sliding layer's 513-544 positions: 9.8 / 8.6 against 8.9 / 8.3.
+// Decodes of spans up to these many positions merge in the kernel: one launch less, which is what a step submitted from the
+// host wants. On the GPU fl_attn and a merge are faster: one token on a full layer at 60 / 250 / 370 positions, fused
+// against two launches, 7.8 / 9.0 / 9.1 against 6.6 / 7.0 / 7.5 us (f32) and 7.5 / 8.3 / 8.3 against 6.4 / 6.8 / 7.3 (f16),
+// a whole step of a sliding and a full layer at 250 positions 31.7 against 27.1 and 30.2 against 26.7. But the host takes
+// 30.9 us to submit the step's eight launches and 35.2 for ten, and a step after the other takes 33.6 against 35.1 us (f32;
+// f16 32.3 / 35.0), one alone 61 / 68. The line lies where two launches of fl_dec16 itself became faster on the GPU: fused
+// against two at 384 / 448 / 768 / 2,048 positions 9.5 / 10.1 / 10.4 / 13.0 against 9.5 / 9.8 / 9.6 / 10.7 us (f32), f16 at 512 /
+// 768 / 2,048 8.8 / 9.0 / 10.4 against 9.0 / 8.7 / 9.2, a sliding layer's 513-544 positions 9.8 / 8.6 against 8.9 / 8.3.
 #ifndef FL_FUSE_SPAN_F32
 #define FL_FUSE_SPAN_F32 384
 #endif
@@ -60,8 +60,10 @@ namespace {
 // shorter ones fl_attn, whose splits of one tile finish sooner. One token on a full layer, us per call, on fl_dec16 (up
 // to 384 positions f32 and 512 f16 with the merge in the kernel) / fl_attn: f32 at 100 / 544 / 1,200 / 2,040 / 3,060
 // positions 8.6 / 9.4 / 9.9 / 10.5 / 11.0 -> 7.1 / 8.0 / 8.2 / 8.4 / 9.8, f16 up to 2,040 7.9 / 8.4 / 8.8 / 9.1 -> 7.0 /
-// 7.1 / 7.5 / 7.9; a sliding layer 9.7 -> 7.9 and 8.8 -> 7.5. Past the line (three tokens on fl_attn against one on
-// fl_dec16): f32 at 5,000 12.6 against 11.7, f16 at 2,500 9.9 against 9.4.
+// 7.1 / 7.5 / 7.9; a sliding layer 9.7 -> 7.9 and 8.8 -> 7.5. Two tokens, keys from HBM, f32 at 520 / 1,000 / 2,040 / 3,050
+// 10.2 / 10.0 / 11.1 / 11.7 -> 8.3 / 8.5 / 9.7 / 10.9, f16 at 520 / 1,000 / 2,040 9.4 / 9.0 / 9.6 -> 7.8 / 7.9 / 8.9; a
+// sliding layer 10.2 -> 8.3 and 9.5 -> 7.9. Past the line (three tokens on fl_attn against one on fl_dec16): f32 at 5,000
+// 12.6 against 11.7, f16 at 2,500 9.9 against 9.4.
 #ifndef FL_DEC_SPAN_F32
 #define FL_DEC_SPAN_F32 3072
 #endif
@@ -1061,17 +1063,14 @@ Plan plan(int fmt, int pos0, int T, int win) {
     int nrb = (T + 3) / 4;
     int nch, blk = 4;
     int fused = 0;
-    if (T <= 2 && span <= (fmt == 1 ? FL_FUSE_SPAN_F32 : FL_FUSE_SPAN_F16)) {  // fl_dec16 merging its own partials: one
-        // launch less; fl_attn and a merge take 7.5 against 9.1 us back to back at 250 positions, but a whole step (32.6
-        // us, a sliding and a full layer) 36.1
+    if (T <= 2 && span <= (fmt == 1 ? FL_FUSE_SPAN_F32 : FL_FUSE_SPAN_F16)) {  // fl_dec16 merging its own partials
         blk = T;
         nch = span / FL_FUSE_SPLIT;
         nch = nch > FL_FUSE_NCH ? FL_FUSE_NCH : nch;
         fused = 1;
     } else if (T <= 2 && span > (fmt == 1 ? FL_DEC_SPAN_F32 : FL_DEC_SPAN_F16)) {  // fl_dec16
         blk = T;
-        nch = span / FL_DEC_SPLIT;
-        nch = nch > FL_DEC_NCH ? FL_DEC_NCH : nch;
+        nch = FL_DEC_NCH;
     } else {
         // 3 tokens and more, and short spans: kernel and splits with the least modelled time (0.01 us), tiles per split
         // against what each split adds in partials and merge. fl_pf (32-token blocks, at most about one work-group per

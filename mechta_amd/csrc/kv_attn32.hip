@@ -346,7 +346,8 @@ Attn32Plan attn32_plan(int T, int n, int start) {
     // windows one (up to 64 tiles: the partials of the smallest store, 4,096 positions, hold 66 splits), two or three,
     // which still leaves at most one work-group per CU: a decode of one / four tokens on four and on these at 200 / 700 /
     // 4,096 / 12,000 positions 19.0 / 15.6 / 14.3 / 17.5 and 19.7 / 16.3 / 16.9 / 19.6 -> 7.9 / 8.2 / 10.9 / 15.1 and
-    // 8.6 / 8.9 / 13.0 / 18.8 us. Every work-group holds keys of every row, so the merge reads all (span 0)
+    // 8.6 / 8.9 / 13.0 / 18.8 us. The merge reads every partial (span 0): the last work-group's one tile may hold only keys
+    // that earlier tokens do not see (4 tokens at 62 positions: key 64), and such rows' m = -inf, l = 0 weigh 0 there
     const int kend = n + T - 1;
     const int keys = kend - start / TILE * TILE, tiles = (keys + TILE - 1) / TILE;
     const int per = tiles <= 64 ? 1 : tiles <= 256 ? 2 : (tiles + 127) / 128;
