@@ -57,11 +57,11 @@ __global__ void __launch_bounds__(NTH, NWV == 4 ? 2 : 1) attn_f32(const float* _
                                                 float* __restrict__ part, const float* __restrict__ akn,
                                                 const float* __restrict__ av, const float* __restrict__ atab, int apos,
                                                 int antok) {
-    // XCD order only where each XCD gets as many work-groups: no two share keys here (one token block), and a grid that is
-    // no multiple of 8, in it, takes longer (1 token at 30,000 positions, 468 work-groups: 30.3 against 28.7 us; 2: 31.8
-    // against 30.8)
+    // XCD order, 0.1-0.4 us faster than launch order on grids of up to about 350 (neighbouring tiles of a kv head then stream
+    // into one XCD), but not for larger ones that are no multiple of 8: 1 token at 25,500 / 30,000 positions (398 / 468
+    // work-groups) 28.8 / 30.3 us in it, 27.4 / 28.7 in launch order, 2 tokens 30.2 / 31.8 against 29.3 / 30.8
     const int G = gridDim.x, L = blockIdx.x;
-    const int W = G % NXCD == 0 ? xcd_order(L, G) : L;
+    const int W = G % NXCD == 0 || G <= 384 ? xcd_order(L, G) : L;
     const int ncg = nch - c0;
     const int rb = W % nrb, c = c0 + (W / nrb) % ncg, kvh = W / nrb / ncg;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, s = lane >> 5, r32 = lane & 31;
